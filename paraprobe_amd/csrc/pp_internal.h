@@ -40,6 +40,10 @@ struct Row {
     int16_t dy, dz, dxm, pad;
 };
 
+// LDS words of the k-th category extraction's windows (one row of 64 uint16
+// per wavefront)
+constexpr int kWinWords = kWaves * kWave / 2;
+
 // Row::pad flags of the symmetric rows: the part of the own row before the
 // own cell (x < cx), or after it (x > cx)
 constexpr int16_t kRowBefore = 1;
@@ -178,6 +182,16 @@ struct JobDev {
     const uint32_t *cellstart_o;
     const uint2 *xsplit_o;
     int xbits_o;
+    // The other center types whose pairs with sym_type are counted from its
+    // tiles (bit set over target slots; their ions lie in list O, s2_o being
+    // its ion2surf): a pair of a center of sym_type and a center of such a
+    // type has one squared distance, so the tile of the former adds it to
+    // both types' pair-count rows (xrow[type]: the words from the tile's own
+    // rows to the row (type, sym_type), or -1).  Tiles of these types read
+    // list S only for its non-centers and their kNN range, then list O.
+    uint32_t sym_minor;
+    const float *s2_o;
+    const int32_t *xrow;
 };
 
 } // namespace pp

@@ -541,7 +541,7 @@ hipError_t launch_typecount(const uint8_t *type, uint64_t n, uint32_t *counts, h
 // query kernel
 
 struct Lay {
-    int edges, envoff, trgslot, kinfo, ckoff, kidx, win, rows, rowpre, cen, meta, P, H, total;
+    int edges, envoff, xrow, kinfo, ckoff, kidx, win, rows, rowpre, cen, meta, P, H, total;
 };
 
 __host__ __device__ inline int al4(int x) { return (x + 3) & ~3; }
@@ -551,7 +551,7 @@ __host__ __device__ inline int al4(int x) { return (x + 3) & ~3; }
 // per-center histograms of maxHK words.
 __host__ __device__ inline Lay make_layout(int T, int c16, int mode, int maxC, int maxE,
                                            int maxTrg, int maxKmax, int maxRows, int maxHK,
-                                           int ntypes)
+                                           int maxP, int ntypes)
 {
     Lay L;
     int o = 0;
@@ -559,25 +559,29 @@ __host__ __device__ inline Lay make_layout(int T, int c16, int mode, int maxC, i
     o += mode == 2 ? 0 : al4(maxC);
     L.envoff = o;  // per type id below ntypes
     o += al4(ntypes);
-    L.trgslot = o;  // unused: tiles carry their center type
+    L.xrow = o;  // per type id: its row against sym_type among the pair counts, or -1
+    o += mode == 0 ? al4(ntypes) : 0;
     L.kinfo = o;
     o += mode == 2 ? 2 * al4(ntypes) : 0;
     L.ckoff = o;
     o += mode == 2 ? kMaxEnv : 0;
     L.kidx = o;  // maxKmax: the largest kmax of the jobs whose k are not 1..kmax
     o += mode && maxKmax ? al4(maxKmax + 2) : 0;
-    L.win = o;  // per wavefront: the k window of the k-th category extraction (uint16)
-    o += mode ? kWaves * kWave / 2 : 0;
     L.rows = o;  // per row its first and end candidate
     o += al4(2 * maxRows);
     L.rowpre = o;  // per row its first index in the rows' concatenation
     o += al4(maxRows + 1);
+    // after the main loop these words hold the tile's tasks and, at their
+    // end, per wavefront the k window of the k-th category extraction (uint16)
+    if (mode && o < L.rows + kWinWords + 24)
+        o = L.rows + kWinWords + 24;
+    L.win = mode ? o - kWinWords : o;
     L.cen = o;
     o += 4 * T;
     L.meta = o;
     o += al4(2 * T);
     L.P = o;
-    o += al4(maxE * maxC);  // pair counts of one center type (tiles hold one type)
+    o += al4(maxP);  // pair counts of one center type (tiles hold one type)
     L.H = o;
     const int hc = c16 ? (T + 1) / 2 : T;
     o += mode == 1 ? al4(hc * maxE * maxC) : mode == 2 ? al4(hc * maxHK) : 0;
@@ -586,9 +590,10 @@ __host__ __device__ inline Lay make_layout(int T, int c16, int mode, int maxC, i
 }
 
 size_t query_lds_bytes(int T, int c16, int mode, int maxC, int maxE, int maxTrg, int maxKmax,
-                       int maxRows, int maxHK, int ntypes)
+                       int maxRows, int maxHK, int maxP, int ntypes)
 {
-    return (size_t)make_layout(T, c16, mode, maxC, maxE, maxTrg, maxKmax, maxRows, maxHK, ntypes)
+    return (size_t)make_layout(T, c16, mode, maxC, maxE, maxTrg, maxKmax, maxRows, maxHK, maxP,
+                               ntypes)
                .total *
            4u;
 }
@@ -601,7 +606,7 @@ struct QArgs {
     uint32_t first_tile, end_tile;
     uint32_t grab;
     int njobs;
-    int maxC, maxE, maxTrg, maxKmax, maxRows, maxHK;
+    int maxC, maxE, maxTrg, maxKmax, maxRows, maxHK, maxP;
     int ntypes;  // type ids of the launch's candidates are below this
 };
 
@@ -642,6 +647,10 @@ typedef __attribute__((address_space(1))) const fvec4 gfvec4;
 template <bool B>
 struct CFlag {
     static constexpr bool value = B;
+};
+template <int I>
+struct CInt {
+    static constexpr int value = I;
 };
 
 typedef __attribute__((address_space(1))) uint16_t gu16;
@@ -746,9 +755,10 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
     extern __shared__ uint32_t lds[];
     __shared__ uint32_t s_g, s_ctot;
     const Lay L = make_layout(T, C16, MODE, a.maxC, a.maxE, a.maxTrg, a.maxKmax, a.maxRows,
-                              a.maxHK, a.ntypes);
+                              a.maxHK, a.maxP, a.ntypes);
     uint32_t *s_edges = lds + L.edges;
     int32_t *s_envoff = (int32_t *)(lds + L.envoff);
+    int32_t *s_xrow = (int32_t *)(lds + L.xrow);
     int2 *s_kinfo = (int2 *)(lds + L.kinfo);
     int32_t *s_ckoff = (int32_t *)(lds + L.ckoff);
     int32_t *s_kidx = (int32_t *)(lds + L.kidx);
@@ -803,6 +813,20 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                         if (v)
                             global_add(&dst[i], (unsigned long long)v);
                     }
+                    if (MODE == 0 && cur % kMaxTrg == P0.sym_slot) {
+                        // the rows (other center type, sym_type)
+                        int k = n;
+                        const int es = P0.envoff[P0.sym_type];
+                        for (uint32_t w = P0.sym_minor; w; w &= w - 1u, k += P0.C) {
+                            unsigned long long *dx =
+                                P0.P + (size_t)__builtin_ctz(w) * n + (size_t)es;
+                            for (int i = tid; i < P0.C; i += kBlock) {
+                                const uint32_t v = s_P[k + i];
+                                if (v)
+                                    global_add(&dx[i], (unsigned long long)v);
+                            }
+                        }
+                    }
                 }
                 if (lane == 0 && inball)
                     atomicAdd(&P0.stats[0], inball);
@@ -822,6 +846,9 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                         s_edges[i] = J.edges[i];
                 for (int i = tid; i < a.ntypes; i += kBlock)
                     s_envoff[i] = J.envoff[i];
+                if (MODE == 0)
+                    for (int i = tid; i < a.ntypes; i += kBlock)
+                        s_xrow[i] = J.xrow[i];
                 if (HY) {
                     for (int i = tid; i < 2 * a.ntypes; i += kBlock)
                         ((int32_t *)s_kinfo)[i] = J.kinfo[i];
@@ -832,7 +859,8 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                     for (int i = tid; i <= J.kmax; i += kBlock)
                         s_kidx[i] = J.kidx_of_k ? J.kidx_of_k[i] : -1;
             }
-            const int n = J.E * J.C;
+            const int n =
+                (J.E + (MODE == 0 && ts == J.sym_slot ? __builtin_popcount(J.sym_minor) : 0)) * J.C;
             for (int i = tid; i < n; i += kBlock)
                 s_P[i] = 0u;
             cur = pkey;
@@ -847,10 +875,12 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
         const int C = J.C, E = J.E, EC = E * C;
         const int HK = HY ? J.HK : 0;
         const int nrows = J.nrows;
-        // symmetric pair counting for this tile's center type: its own-type
-        // candidates along srows[0, s_ns) of list S, the others along
-        // srows[s_ns, nsrows) of list O
-        const bool sym = !PC && ts == J.sym_slot;
+        // symmetric pair counting: the candidates of sym_type along srows[0,
+        // s_ns) of list S, the others along srows[s_ns, nsrows) of list O, in
+        // the tiles of sym_type and (minor) of the types whose pairs with its
+        // centers its tiles count
+        const bool minor = MODE == 0 && ((J.sym_minor >> ts) & 1u) != 0u;
+        const bool sym = !PC && (ts == J.sym_slot || minor);
         const int nrt = sym ? J.nsrows : nrows;
         const Row *rtab = sym ? J.srows : J.rows;
         const int cx = (int)(key % (uint32_t)J.nx);
@@ -931,10 +961,11 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                 };
                 cut(J.reach * J.reach);
                 const uint32_t kr = ((uint32_t)z * (uint32_t)J.ny + (uint32_t)y) * (uint32_t)J.nx;
-                if (inS && r >= 1 && r < J.s_nb1 && x0 <= x1) {
-                    // a row before the own cell: the pairs with centers there
+                if (inS && (minor || (r >= 1 && r < J.s_nb1)) && x0 <= x1) {
+                    // a row before the own cell (for a minor type's tile
+                    // every row): the pairs with centers there
                     // are counted from those centers' tiles, so a cell whose
-                    // own-type ions are all centers is needed only within the
+                    // ions of sym_type are all centers is needed only within the
                     // kNN reach.  The row keeps the cells holding a non-center
                     // (fa .. fb) and the kNN reach: their hull, trimmed at its
                     // ends as the full-reach row (as the kNN reach when no
@@ -1055,9 +1086,10 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
             uint32_t *s_acc = PC ? s_H : s_P;
             const uint32_t ctot = rfl(s_ctot);
             unsigned long long my_in = 0;
-            // symmetric tiles: the own type's pair-count row and kNN-range
-            // entries (uniform), and the candidate indices where the cells
+            // symmetric tiles: the pair-count row and kNN-range entries of
+            // sym_type (uniform), and the candidate indices where the cells
             // before the own cell (sb1) and after it (sb2) start in list S
+            // (a minor type's tile takes all of list S as before)
             int woff_t = 0, kof_t = 0;
             float kthr_t = -1.0f;
             uint32_t sb1 = 0, sb2 = 0;
@@ -1068,8 +1100,8 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                     kof_t = (int)rfl((uint32_t)ki.x);
                     kthr_t = __int_as_float((int)rfl((uint32_t)ki.y));
                 }
-                sb1 = rfl(s_rowpre[1]);
-                sb2 = rfl(s_rowpre[J.s_nb1]);
+                sb1 = minor ? 0u : rfl(s_rowpre[1]);
+                sb2 = rfl(s_rowpre[minor ? J.s_ns : J.s_nb1]);
             }
             // One pass over rows [rlo, rhi) of list pos, whose candidates
             // are clo .. chi - 1 of the tile's concatenation.  Each
@@ -1079,11 +1111,16 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
             // Every lane keeps its own cursor: row r, index j, row end re
             // (r == rhi: past the last row).  Two chunks alternate, so that
             // the load of the next is in flight while one is evaluated
-            // against the T centers.  SYMF: the own-type pass of a symmetric
-            // tile.
-            auto sweep = [&](auto SYMF, const gfvec4 *__restrict__ pos, int rlo, int rhi,
+            // against the T centers.  KIND 1: the pass over list S of a
+            // symmetric tile; 2: over list O of a sym_type tile that also
+            // counts its pairs with the centers of other types for them; 0:
+            // any other.
+            auto sweep = [&](auto KIND, const gfvec4 *__restrict__ pos, int rlo, int rhi,
                              uint32_t clo, uint32_t chi) {
-            constexpr bool SY = !PC && decltype(SYMF)::value;
+            constexpr bool SY = !PC && decltype(KIND)::value == 1;
+            constexpr bool XS = MODE == 0 && decltype(KIND)::value == 2;
+            typedef __attribute__((address_space(1))) const float gfloat;
+            const gfloat *s2o = XS ? rflp((const gfloat *)J.s2_o) : nullptr;
             const int nch = (int)((chi - clo + kWave - 1) / kWave);
             const int qa = (int)rfl((uint32_t)(wid * nch / kWaves));
             const int qb = (int)rfl((uint32_t)((wid + 1) * nch / kWaves));
@@ -1108,8 +1145,10 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                 }
             }
             // the chunk at the cursor (lanes past the last row load ion 0)
-            auto fetch = [&](bool &ok) {
+            auto fetch = [&](bool &ok, float &s2) {
                 ok = r < rhi;
+                if (XS)
+                    s2 = s2o[j];
                 return load_g4(pos, j);
             };
             // the next chunk: 64 candidates on, across row ends (empty rows
@@ -1129,10 +1168,12 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                     re = s_rows[2 * r + 1];
                 }
             };
-            auto body = [&](float4 p, const bool ok, int q) {
+            auto body = [&](float4 p, float s2, const bool ok, int q) {
                 // keep every use of this chunk's data below this point, so the
                 // wait for its load is not hoisted into the prefetch of the next
                 asm volatile("" : "+v"(p.x), "+v"(p.y), "+v"(p.z), "+v"(p.w));
+                if (XS)
+                    asm volatile("" : "+v"(s2));
                 const float px = ok ? p.x : __builtin_nanf("");
                 // (the own-type pass of a symmetric tile knows the type, and
                 // its w holds ion2surf)
@@ -1153,6 +1194,10 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                 asm volatile("" : "+s"(cin));
                 // this candidate's pair-count row (only dereferenced when envok)
                 uint32_t *acc_row = (PC ? s_H : s_P) + woff;
+                // and its own type's row against sym_type, when it is a center
+                const int xr = XS ? s_xrow[ptype] : 0;
+                const bool xadd = XS && xr >= 0 && s2 >= R2;
+                uint32_t *x_row = s_P + xr;
                 if (PC) {
                     // 1) all T squared distances (the reference's FP32 expression)
                     float d2[T];
@@ -1244,6 +1289,9 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                                 __hip_atomic_fetch_add(acc_row + cat, 1u,
                                                        __ATOMIC_RELAXED,
                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
+                                if (xadd)
+                                    __hip_atomic_fetch_add(x_row + cat, 1u, __ATOMIC_RELAXED,
+                                                           __HIP_MEMORY_SCOPE_WORKGROUP);
                             }
                         }
                     }
@@ -1335,28 +1383,34 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
             // make the wait for one chunk wait for the other too
             bool oka = false, okb = false;
             float4 pa = make_float4(0.f, 0.f, 0.f, 0.f), pb = pa;
+            float s2a = 0.f, s2b = 0.f;
             if (qa < qb)
-                pa = fetch(oka);
+                pa = fetch(oka, s2a);
             for (int q = qa; q < qb; q += 2) {
                 if (q + 1 < qb)
                     advance();
-                pb = fetch(okb);
-                body(pa, oka, q);
+                pb = fetch(okb, s2b);
+                body(pa, s2a, oka, q);
                 if (q + 2 < qb)
                     advance();
-                pa = fetch(oka);
+                pa = fetch(oka, s2a);
                 if (q + 1 < qb)
-                    body(pb, okb, q + 1);
+                    body(pb, s2b, okb, q + 1);
             }
             };
             if (sym) {
                 const uint32_t bs = rfl(s_rowpre[J.s_ns]);
                 const int ns = (int)rfl((uint32_t)J.s_ns);
-                sweep(CFlag<true>(), rflp((const gfvec4 *)J.pos_s), 0, ns, 0u, bs);
-                if (ns < nrt)
-                    sweep(CFlag<false>(), rflp((const gfvec4 *)J.pos_o), ns, nrt, bs, ctot);
+                sweep(CInt<1>(), rflp((const gfvec4 *)J.pos_s), 0, ns, 0u, bs);
+                if (ns < nrt) {
+                    if (MODE == 0 && !minor && J.sym_minor != 0u)
+                        sweep(CInt<MODE == 0 ? 2 : 0>(), rflp((const gfvec4 *)J.pos_o), ns, nrt, bs,
+                              ctot);
+                    else
+                        sweep(CInt<0>(), rflp((const gfvec4 *)J.pos_o), ns, nrt, bs, ctot);
+                }
             } else {
-                sweep(CFlag<false>(), rflp((const gfvec4 *)J.pos), 0, nrows, 0u, ctot);
+                sweep(CInt<0>(), rflp((const gfvec4 *)J.pos), 0, nrows, 0u, ctot);
             }
             inball += my_in;
         }
@@ -1397,8 +1451,9 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
         // here rather than by each center's wave in series, into the stencil
         // rows' words (free until the next tile) as far as they hold them
         const int Lt = (int)J.trg_ntask[ts];
-        // (the rows' starts and prefix hold L.cen - L.rows words)
-        const int Ls = Lt < (L.cen - L.rows) / 3 ? Lt : (L.cen - L.rows) / 3;
+        // (the rows' starts and prefix hold L.win - L.rows words before the
+        // extraction's windows)
+        const int Ls = Lt < (L.win - L.rows) / 3 ? Lt : (L.win - L.rows) / 3;
         uint32_t *s_task = s_rows;  // (the main loop's closing barrier freed them)
         for (int l = tid; l < Ls; l += kBlock) {
             const uint32_t tk = J.trg_tasks[ts * J.lmax + l];
@@ -1615,7 +1670,7 @@ template <int T, bool C16, int MODE>
 static hipError_t launch_query_t(const QueryLaunch &q, hipStream_t s)
 {
     const size_t lds = query_lds_bytes(T, C16, MODE, q.maxC, q.maxE, q.maxTrg, q.maxKmax,
-                                       q.maxRows, q.maxHK, q.ntypes);
+                                       q.maxRows, q.maxHK, q.maxP, q.ntypes);
     QArgs a;
     a.jobs = q.jobs;
     a.tile_off = q.tile_off;
@@ -1632,6 +1687,7 @@ static hipError_t launch_query_t(const QueryLaunch &q, hipStream_t s)
     a.ntypes = q.ntypes;
     a.maxRows = q.maxRows;
     a.maxHK = q.maxHK;
+    a.maxP = q.maxP;
     hipError_t e = hipFuncSetAttribute((const void *)k_query<T, C16, MODE>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess)
