@@ -838,38 +838,54 @@ void layout_outputs(JobRun &r, Carver &m)
 // The lists one preparation of a run builds (sized for every job of the
 // run; a rerun of some of them fits too).
 struct PrepArena {
-    uint64_t E = 0, Ec = 0, nion = 0;
+    uint64_t E = 0, Ec = 0, nc = 0, nion = 0;
+    uint64_t nions = 0;  // ions of all segments
     int nseg = 0, njobs = 0;
-    uint32_t *flags = nullptr, *cpos = nullptr, *centers = nullptr, *ntile = nullptr,
-             *toff = nullptr, *ws = nullptr;
+    PrepLists l{};
+    uint32_t *centers = nullptr;
     Tile *tiles = nullptr;
     PrepSeg *segs = nullptr;
     int32_t *jseg = nullptr;
     PrepJobStat *js = nullptr;
 };
 
+uint64_t prep_pad(uint64_t n) { return (n + kPrepTile - 1) / kPrepTile * kPrepTile; }
+
 void size_prep(PrepArena &a, const std::vector<JobRun> &runs)
 {
-    a.E = a.Ec = a.nion = 0;
+    a.E = a.Ec = a.nc = a.nion = a.nions = 0;
     a.nseg = 0;
     a.njobs = (int)runs.size();
     for (const JobRun &r : runs) {
         const uint64_t k = (uint64_t)r.plan.ntrg;
-        a.E += (uint64_t)r.cloud->n * k;
-        a.Ec += (uint64_t)r.ncells * k;
+        a.E += prep_pad(r.cloud->n) * k;
+        a.Ec += prep_pad(r.ncells) * k;
+        a.nc += (uint64_t)r.ncells * k;
         a.nion += r.cloud->n;
+        a.nions += (uint64_t)r.cloud->n * k;
         a.nseg += r.plan.ntrg;
     }
 }
 
-void layout_prep(PrepArena &a, Carver &m)
+// (fixed: the no-allocation scratch, whose limit on a job -- about 32 bytes an
+// ion -- callers plan by: there the lists take the room of 4-byte flags,
+// positions, tile counts and offsets and their scan's workspace, as they did)
+void layout_prep(PrepArena &a, Carver &m, bool fixed)
 {
-    a.flags = m.take<uint32_t>(a.E + 1);
-    a.cpos = m.take<uint32_t>(a.E + 1);
+    Carver room(nullptr);
+    room.off = m.off;
+    if (fixed)
+        for (uint64_t words : {a.nions + 1, a.nions + 1, a.nc + 1, a.nc + 1,
+                               (uint64_t)scan_workspace_words(std::max(a.nions, a.nc))})
+            room.take<uint32_t>(words);
+    const PrepWords w = prep_words(a.E, a.Ec, a.nc);
+    a.l.bits = (uint64_t *)m.take<uint32_t>(w.bits);
+    a.l.wpos = m.take<uint32_t>(w.wpos);
+    a.l.boff = m.take<uint32_t>(w.boff);
+    a.l.tpre = m.take<uint32_t>(w.tpre);
+    a.l.toff = m.take<uint32_t>(w.toff);
+    m.off = std::max(m.off, room.off);
     a.centers = m.take<uint32_t>(a.nion + 1);
-    a.ntile = m.take<uint32_t>(a.Ec + 1);
-    a.toff = m.take<uint32_t>(a.Ec + 1);
-    a.ws = m.take<uint32_t>(prep_workspace_words(a.E, a.Ec));
     a.tiles = m.take<Tile>(a.nion + 1);  // at most one tile per center
     a.segs = m.take<PrepSeg>((size_t)std::max(a.nseg, 1));
     a.jseg = m.take<int32_t>((size_t)a.njobs + 1);
@@ -881,7 +897,7 @@ size_t prep_bytes(uint64_t n, uint64_t nc, int ntrg)
 {
     const uint64_t k = (uint64_t)std::max(ntrg, 1);
     return (size_t)(n * k * 8 + n * 4 + n * 16 + nc * k * 8 +
-                    4 * prep_workspace_words(n * k, nc * k) + 4096);
+                    4 * scan_workspace_words(std::max(n * k, nc * k)) + 4096);
 }
 
 // The host image of a job's device tables.
@@ -932,7 +948,7 @@ pp_status prep_run(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std::ve
         return PP_OK;
     std::vector<PrepSeg> segs;
     std::vector<int32_t> jseg(nj + 1, 0);
-    uint64_t E = 0, Ec = 0;
+    uint64_t E = 0, Ec = 0, nc = 0, jblocks = 0;
     for (int q = 0; q < nj; ++q) {
         JobRun &r = runs[ids[q]];
         const JobPlan &p = r.plan;
@@ -948,20 +964,25 @@ pp_status prep_run(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std::ve
             g.g = r.cl->g;
             g.ion0 = E;
             g.cell0 = Ec;
+            g.tp0 = nc;
             g.n = (uint32_t)r.cloud->n;
             g.nc = (uint32_t)r.ncells;
+            g.jblk0 = (uint32_t)jblocks;
             g.nrows = (int)r.rows.size();
             g.R2 = p.R2;
             g.slot = slot;
             g.T = r.T_req;
             g.job = q;
             segs.push_back(g);
-            E += r.cloud->n;
-            Ec += r.ncells;
+            E += prep_pad(r.cloud->n);
+            Ec += prep_pad(r.ncells);
+            nc += r.ncells;
         }
+        if (p.ntrg > 0)
+            jblocks += prep_pad(r.cloud->n) / kPrepTile;
     }
     jseg[nj] = (int32_t)segs.size();
-    if (E > a.E || Ec > a.Ec || (int)segs.size() > a.nseg || nj > a.njobs)
+    if (E > a.E || Ec > a.Ec || nc > a.nc || (int)segs.size() > a.nseg || nj > a.njobs)
         return fail(c, PP_ERR_HIP, "internal: preparation larger than its arena");
     hipStream_t s = sl.stream;
     if (!segs.empty())
@@ -975,12 +996,9 @@ pp_status prep_run(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std::ve
     L.njobs = nj;
     L.E = E;
     L.Ec = Ec;
-    L.flags = a.flags;
-    L.cpos = a.cpos;
+    L.jblocks = (uint32_t)jblocks;
+    L.l = a.l;
     L.centers = a.centers;
-    L.ntile = a.ntile;
-    L.toff = a.toff;
-    L.ws = a.ws;
     L.tiles = a.tiles;
     L.js = a.js;
     std::vector<PrepJobStat> js(nj);
@@ -2059,7 +2077,7 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
         }
         for (int i = 0; i < njobs; ++i)
             runs[i].flags = m.take<uint32_t>(runs[i].cloud->n + 1);
-        layout_prep(pa, m);
+        layout_prep(pa, m, sl.fixed != nullptr);
     };
     char *out0 = nullptr, *out1 = nullptr;
     Carver m0(nullptr);

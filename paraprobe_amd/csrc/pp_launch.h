@@ -67,7 +67,8 @@ hipError_t launch_occupancy(const float *xyz, uint64_t n, OccGrid g, uint8_t *oc
 // Centers and tiles of a run of jobs in one pass (pp_prep.hip).  One segment
 // per (job, center type slot), a job's segments consecutive; segment q's ions
 // occupy [ion0, ion0 + n) of the run's ion space and its cells
-// [cell0, cell0 + nc) of the cell space.
+// [cell0, cell0 + nc) of the cell space, each start a multiple of kPrepTile.
+constexpr uint32_t kPrepTile = 2048;
 struct PrepSeg {
     const float4 *pos;         // the job's cell-sorted ions (x, y, z, type bits)
     const float *s2;           // their ion2surf
@@ -77,11 +78,24 @@ struct PrepSeg {
     const Row *rows;           // the job's stencil rows
     GridGeom g;
     uint64_t ion0, cell0;
+    uint64_t tp0;              // its cells' start in PrepLists::tpre (not padded)
     uint32_t n, nc;
+    uint32_t jblk0;            // the job's first block of kPrepTile ions (ions counted once per job)
     int nrows;
     float R2;                  // fl32(R * R): considered iff ion2surf >= R2
     int slot, T, job;
 };
+// The run's temporary lists: a bit per element of the ion space, the centers
+// before each 64 of them in their block, the centers before each block (and
+// the total); the tiles before each cell in its block and before each block.
+struct PrepLists {
+    uint64_t *bits;
+    uint32_t *wpos, *boff, *tpre, *toff;
+};
+struct PrepWords {
+    size_t bits, wpos, boff, tpre, toff;  // sizes in 4-byte words
+};
+PrepWords prep_words(uint64_t E, uint64_t Ec, uint64_t nc);  // nc: cells of all segments
 // Per job: its centers [center0, center0 + centers) of the run's center list,
 // its tiles [tile0, tile0 + tiles) of the run's tile list, and the largest
 // stencil candidate count of a cell with centers.
@@ -93,17 +107,13 @@ struct PrepLaunch {
     int nseg;
     const int32_t *jseg;       // device [njobs + 1]: job j's segments [jseg[j], jseg[j + 1])
     int njobs;
-    uint64_t E, Ec;            // sizes of the ion and cell spaces
-    uint32_t *flags;           // E
-    uint32_t *cpos;            // E + 1: exclusive scan of flags (center positions)
+    uint64_t E, Ec;            // sizes of the ion and cell spaces (multiples of kPrepTile)
+    uint32_t jblocks;          // blocks of kPrepTile ions, each job's ions counted once
+    PrepLists l;
     uint32_t *centers;         // the run's center list (job-local sorted ion indices)
-    uint32_t *ntile;           // Ec
-    uint32_t *toff;            // Ec + 1
-    uint32_t *ws;              // prep_workspace_words(E, Ec)
     Tile *tiles;               // the run's tiles (Tile::first indexes centers, Tile::job the job)
     PrepJobStat *js;           // device [njobs]
 };
-size_t prep_workspace_words(uint64_t E, uint64_t Ec);
 hipError_t launch_prep(const PrepLaunch &p, hipStream_t s);
 
 // Query launch over all jobs of a launch.

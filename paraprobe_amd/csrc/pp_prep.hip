@@ -7,12 +7,23 @@
 // whose type has slot q.slot and whose ion2surf is at least fl32(R^2)
 // (src/PARAPROBE_SolverHdl.cpp:3846-3860), or the ions a rerun selection
 // flags.  All segments' ion ranges are laid end to end (the ion space, ion0
-// onwards for segment q) and so are their cell ranges (the cell space,
-// cell0 onwards): one flag pass, one exclusive scan and one compaction give
-// the run's center list (segment after segment, each in cell order); one
-// count pass, one scan and one write pass give its tiles -- up to T centers
-// of one segment in one cell, first center as an index into the run's center
-// list -- and each job's largest stencil candidate count.
+// onwards for segment q), each padded to whole blocks of kPrepTile, and so are
+// their cell ranges (the cell space, cell0 onwards), so that no block spans
+// segments.  Five launches: one pass over each job's ions sets a bit per
+// (segment, ion) and counts it per 64 ions and per block for all of the job's
+// segments at once; a one-block scan turns the block counts into offsets;
+// then the compaction into the run's center list (segment after segment, each
+// in cell order) and, in the same launch, the tiles per cell with their
+// in-block prefix; a second scan; and the tiles -- up to T centers of one
+// segment in one cell, first center as an index into the run's center list --
+// with each job's largest stencil candidate count and its parts of the lists.
+//
+// What bounds it: reading 20 bytes an ion once (it was once per segment, with
+// a 4-byte flag and a 4-byte scanned position for each written and read
+// again), and for small runs the number of launches, 5 instead of 12.  A
+// whole call, before and after: 20,000 ions with three center types 303 and
+// 283 us, a batch of 24 jobs of 50,000 to 2,000,000 ions 7.73 and 7.20 ms, 100
+// million ions with one center type 423 and 415 ms.
 #include "pp_launch.h"
 
 namespace pp {
@@ -20,83 +31,205 @@ namespace pp {
 namespace {
 
 constexpr int kPrepBlock = 256;
+constexpr int kPrepItems = kPrepTile / kPrepBlock;
+constexpr int kPrepWords = kPrepTile / 64;  // 64-ion words of a block
 
-// The segment holding element e of a space whose segment starts are
-// start(q): thread 0 of the block finds the block's first element's segment
-// by bisection, every thread then steps forward (elements of one block span
-// few segments).
+// the last k in [0, n) with start(k) <= b (starts ascending, start(0) <= b),
+// by the block's first thread
 template <typename Start>
-__device__ inline int seg_of(uint64_t e, uint64_t block_first, int nseg, Start start,
-                             int *s_first)
+__device__ inline int find_last(uint64_t b, int n, Start start, int *s_q)
 {
     if (threadIdx.x == 0) {
-        int lo = 0, hi = nseg;  // start(lo) <= block_first < start(hi)
+        int lo = 0, hi = n;
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
-            if (start(mid) <= block_first)
+            if (start(mid) <= b)
                 lo = mid;
             else
                 hi = mid;
         }
-        *s_first = lo;
+        *s_q = lo;
     }
     __syncthreads();
-    int q = *s_first;
-    while (q + 1 < nseg && start(q + 1) <= e)
-        ++q;
-    return q;
+    return *s_q;
 }
 
-__global__ __launch_bounds__(kPrepBlock) void k_pflags(const PrepSeg *__restrict__ segs, int nseg,
-                                                        uint64_t E, uint32_t *__restrict__ flags)
+// centers before element e of the ion space
+__device__ inline uint32_t center_pos(const PrepLists &l, uint64_t e)
 {
-    __shared__ int s_first;
-    const uint64_t b0 = (uint64_t)blockIdx.x * kPrepBlock;
-    const uint64_t e = b0 + threadIdx.x;
-    const int q = seg_of(e < E ? e : E - 1, b0, nseg, [&](int k) { return segs[k].ion0; },
-                         &s_first);
-    if (e >= E)
-        return;
-    const PrepSeg S = segs[q];  // by value: kept in registers, not re-read
-    const uint64_t i = e - S.ion0;
-    const uint32_t t = __float_as_uint(S.pos[i].w) & 0xFFu;
-    const int ts = S.trgslot[t];
-    const bool sel = S.src ? S.src[i] != 0u : (ts >= 0 && S.s2[i] >= S.R2);
-    flags[e] = (sel && ts == S.slot) ? 1u : 0u;
+    uint32_t p = l.boff[e / kPrepTile];
+    if (e % kPrepTile) {  // (at a block's start, or at the space's end, that is all)
+        const uint64_t w = e >> 6;
+        p += l.wpos[w] + (uint32_t)__builtin_popcountll(l.bits[w] & ((1ull << (e & 63)) - 1ull));
+    }
+    return p;
 }
 
-// centers[cpos[e]] = the job-local sorted ion index of every flagged element
+// One block per kPrepTile ions of a job, for all of the job's segments.
+__global__ __launch_bounds__(kPrepBlock) void k_pflags(const PrepSeg *__restrict__ segs,
+                                                        const int32_t *__restrict__ jseg, int njobs,
+                                                        PrepLists l, PrepJobStat *__restrict__ js)
+{
+    __shared__ int s_q;
+    __shared__ uint64_t s_bits[kMaxTrg][kPrepWords];
+    if (blockIdx.x == 0)
+        for (int k = threadIdx.x; k < njobs; k += kPrepBlock)
+            js[k].maxcand = 0u;
+    // (a job without segments starts where the next one does and owns no block)
+    const int j = find_last(blockIdx.x, njobs, [&](int k) {
+        return jseg[k] < jseg[njobs] ? (uint64_t)segs[jseg[k]].jblk0 : ~0ull; }, &s_q);
+    const int q0 = jseg[j], ns = jseg[j + 1] - q0;
+    const PrepSeg S = segs[q0];  // by value: kept in registers, not re-read
+    if (S.n == 0)
+        return;  // no ions at all: the one block is here for the counters
+    const uint32_t b0 = (blockIdx.x - S.jblk0) * (uint32_t)kPrepTile;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x / 64;
+    int ts[kPrepItems];
+#pragma unroll
+    for (int k = 0; k < kPrepItems; ++k) {
+        const uint64_t i = (uint64_t)b0 + (uint64_t)(k * kPrepBlock) + threadIdx.x;
+        ts[k] = -1;
+        if (i < S.n && (S.src ? S.src[i] != 0u : S.s2[i] >= S.R2))
+            ts[k] = S.trgslot[__float_as_uint(S.pos[i].w) & 0xFFu];
+    }
+    // (the segments of a job are its center type slots in order)
+    for (int q = 0; q < ns; ++q) {
+#pragma unroll
+        for (int k = 0; k < kPrepItems; ++k) {
+            const uint64_t m = __ballot(ts[k] == q);
+            if (lane == 0)
+                s_bits[q][k * (kPrepBlock / 64) + wid] = m;
+        }
+    }
+    __syncthreads();
+    static_assert(kPrepWords == 32, "one word per lane of half a wavefront");
+    for (int q = wid; q < ns; q += kPrepBlock / 64) {
+        const uint64_t m = lane < kPrepWords ? s_bits[q][lane] : 0ull;
+        const uint32_t n = (uint32_t)__builtin_popcountll(m);
+        uint32_t incl = n;
+        for (int d = 1; d < kPrepWords; d <<= 1) {
+            const uint32_t o = (uint32_t)__shfl_up((int)incl, d, 64);
+            if (lane >= d)
+                incl += o;
+        }
+        const uint64_t w = (segs[q0 + q].ion0 + b0) / 64 + (uint64_t)lane;
+        if (lane < kPrepWords) {
+            l.bits[w] = m;
+            l.wpos[w] = incl - n;
+        }
+        if (lane == kPrepWords - 1)
+            l.boff[(segs[q0 + q].ion0 + b0) / kPrepTile] = incl;
+    }
+}
+
+// Exclusive scan of n block counts in place, the total at index n; one block
+// (a block count stands for kPrepTile elements, so there are few).
+__global__ __launch_bounds__(1024) void k_pscan(uint32_t *__restrict__ v, uint32_t n)
+{
+    __shared__ uint32_t s_w[16];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x / 64;
+    uint32_t carry = 0;
+    for (uint32_t b = 0; b < n; b += 4096) {
+        const uint32_t i = b + threadIdx.x * 4u;
+        uint32_t a[4], tot = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            a[k] = i + (uint32_t)k < n ? v[i + (uint32_t)k] : 0u;
+            tot += a[k];
+        }
+        uint32_t incl = tot;
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t o = (uint32_t)__shfl_up((int)incl, d, 64);
+            if (lane >= d)
+                incl += o;
+        }
+        if (lane == 63)
+            s_w[wid] = incl;
+        __syncthreads();
+        uint32_t before = 0, all = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) {
+            const uint32_t x = s_w[w];
+            before += w < wid ? x : 0u;
+            all += x;
+        }
+        uint32_t run = carry + before + incl - tot;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (i + (uint32_t)k < n)
+                v[i + (uint32_t)k] = run;
+            run += a[k];
+        }
+        carry += all;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0)
+        v[n] = carry;
+}
+
+// Blocks below nion: the centers of one block of the ion space (job-local
+// sorted ion indices); the others: the tiles per cell of one block of the
+// cell space, as their prefix in the block and the block's total.
 __global__ __launch_bounds__(kPrepBlock) void k_pcompact(const PrepSeg *__restrict__ segs,
-                                                          int nseg, uint64_t E,
-                                                          const uint32_t *__restrict__ flags,
-                                                          const uint32_t *__restrict__ cpos,
+                                                          int nseg, uint32_t nion, PrepLists l,
                                                           uint32_t *__restrict__ centers)
 {
-    __shared__ int s_first;
-    const uint64_t b0 = (uint64_t)blockIdx.x * kPrepBlock;
-    const uint64_t e = b0 + threadIdx.x;
-    const int q = seg_of(e < E ? e : E - 1, b0, nseg, [&](int k) { return segs[k].ion0; },
-                         &s_first);
-    if (e < E && flags[e])
-        centers[cpos[e]] = (uint32_t)(e - segs[q].ion0);
-}
-
-__global__ __launch_bounds__(kPrepBlock) void k_ptilecount(const PrepSeg *__restrict__ segs,
-                                                            int nseg, uint64_t Ec,
-                                                            const uint32_t *__restrict__ cpos,
-                                                            uint32_t *__restrict__ ntile)
-{
-    __shared__ int s_first;
-    const uint64_t b0 = (uint64_t)blockIdx.x * kPrepBlock;
-    const uint64_t e = b0 + threadIdx.x;
-    const int q = seg_of(e < Ec ? e : Ec - 1, b0, nseg, [&](int k) { return segs[k].cell0; },
-                         &s_first);
-    if (e >= Ec)
+    __shared__ int s_q;
+    __shared__ uint32_t s_w[kPrepBlock / 64];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x / 64;
+    if (blockIdx.x < nion) {
+        const uint64_t e0 = (uint64_t)blockIdx.x * kPrepTile;
+        const int q = find_last(e0, nseg, [&](int k) { return segs[k].ion0; }, &s_q);
+        const uint32_t i0 = (uint32_t)(e0 - segs[q].ion0), off = l.boff[blockIdx.x];
+        for (int k = 0; k < kPrepItems; ++k) {
+            const uint64_t w = e0 / 64 + (uint64_t)(k * (kPrepBlock / 64) + wid);
+            const uint64_t m = l.bits[w];
+            if ((m >> lane) & 1ull)
+                centers[off + l.wpos[w] +
+                        (uint32_t)__builtin_popcountll(m & ((1ull << lane) - 1ull))] =
+                    i0 + (uint32_t)(k * kPrepBlock) + threadIdx.x;
+        }
         return;
+    }
+    const uint32_t cb = blockIdx.x - nion;
+    const uint64_t e0 = (uint64_t)cb * kPrepTile;
+    const int q = find_last(e0, nseg, [&](int k) { return segs[k].cell0; }, &s_q);
     const PrepSeg S = segs[q];
-    const uint64_t c = e - S.cell0;
-    const uint32_t lo = cpos[S.ion0 + S.cellstart[c]], hi = cpos[S.ion0 + S.cellstart[c + 1]];
-    ntile[e] = (hi - lo + (uint32_t)S.T - 1u) / (uint32_t)S.T;
+    const uint64_t c0 = e0 - S.cell0 + (uint64_t)threadIdx.x * kPrepItems;
+    uint32_t cnt[kPrepItems], tot = 0;
+    uint32_t lo = c0 < S.nc ? center_pos(l, S.ion0 + S.cellstart[c0]) : 0u;
+#pragma unroll
+    for (int k = 0; k < kPrepItems; ++k) {
+        cnt[k] = 0;
+        if (c0 + (uint64_t)k < S.nc) {
+            const uint32_t hi = center_pos(l, S.ion0 + S.cellstart[c0 + (uint64_t)k + 1u]);
+            cnt[k] = (hi - lo + (uint32_t)S.T - 1u) / (uint32_t)S.T;
+            lo = hi;
+        }
+        tot += cnt[k];
+    }
+    uint32_t incl = tot;
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)incl, d, 64);
+        if (lane >= d)
+            incl += o;
+    }
+    if (lane == 63)
+        s_w[wid] = incl;
+    __syncthreads();
+    uint32_t run = incl - tot, all = 0;
+    for (int w = 0; w < kPrepBlock / 64; ++w) {
+        run += w < wid ? s_w[w] : 0u;
+        all += s_w[w];
+    }
+#pragma unroll
+    for (int k = 0; k < kPrepItems; ++k) {
+        if (c0 + (uint64_t)k < S.nc)
+            l.tpre[S.tp0 + c0 + (uint64_t)k] = run;
+        run += cnt[k];
+    }
+    if (threadIdx.x == 0)
+        l.toff[cb] = all;
 }
 
 // stencil row rw around cell (cx, cy, cz): its candidate range, empty when
@@ -114,30 +247,47 @@ __device__ inline uint32_t row_count(const Row &rw, int cx, int cy, int cz, cons
 }
 
 // The tiles of every cell with centers, and each job's largest stencil
-// candidate count (a bound on any center's neighbour count).
+// candidate count (a bound on any center's neighbour count); the first block
+// also writes each job's parts of the run's lists.
 __global__ __launch_bounds__(kPrepBlock) void k_ptilewrite(const PrepSeg *__restrict__ segs,
-                                                            int nseg, uint64_t Ec,
-                                                            const uint32_t *__restrict__ cpos,
-                                                            const uint32_t *__restrict__ toff,
+                                                            int nseg,
+                                                            const int32_t *__restrict__ jseg,
+                                                            int njobs, PrepLists l,
                                                             Tile *__restrict__ tiles,
                                                             PrepJobStat *__restrict__ js)
 {
-    __shared__ int s_first;
+    __shared__ int s_q;
     const uint64_t b0 = (uint64_t)blockIdx.x * kPrepBlock;
+    if (blockIdx.x == 0)
+        for (int j = threadIdx.x; j < njobs; j += kPrepBlock) {
+            const int a = jseg[j], b = jseg[j + 1];
+            uint32_t c0 = 0, c1 = 0, t0 = 0, t1 = 0;
+            if (a < b) {
+                // (a segment's blocks are its own, so the next one's offset
+                // is where it ends)
+                const PrepSeg &F = segs[a], &L = segs[b - 1];
+                c0 = l.boff[F.ion0 / kPrepTile];
+                c1 = l.boff[(L.ion0 + L.n + kPrepTile - 1) / kPrepTile];
+                t0 = l.toff[F.cell0 / kPrepTile];
+                t1 = l.toff[(L.cell0 + L.nc + kPrepTile - 1) / kPrepTile];
+            }
+            js[j].center0 = c0;
+            js[j].centers = c1 - c0;
+            js[j].tile0 = t0;
+            js[j].tiles = t1 - t0;
+        }
+    const int q = find_last(b0, nseg, [&](int k) { return segs[k].cell0; }, &s_q);
+    const PrepSeg S = segs[q];  // by value: kept in registers, not re-read
     const uint64_t e = b0 + threadIdx.x;
-    const int q = seg_of(e < Ec ? e : Ec - 1, b0, nseg, [&](int k) { return segs[k].cell0; },
-                         &s_first);
+    const uint64_t c = e - S.cell0;
     // every lane stays to the wave's reduction below (no early return)
     uint32_t tot = 0;
-    int job = 0;
-    if (e < Ec) {
-        const PrepSeg S = segs[q];  // by value: kept in registers, not re-read
-        job = S.job;
-        const uint64_t c = e - S.cell0;
-        const uint32_t lo = cpos[S.ion0 + S.cellstart[c]],
-                       hi = cpos[S.ion0 + S.cellstart[c + 1]];
+    if (c < S.nc) {
+        const uint32_t lo = center_pos(l, S.ion0 + S.cellstart[c]),
+                       hi = center_pos(l, S.ion0 + S.cellstart[c + 1]);
         if (hi > lo) {
-            const uint32_t T = (uint32_t)S.T, cnt = hi - lo, t0 = toff[e];
+            const uint32_t T = (uint32_t)S.T, cnt = hi - lo;
+            const uint32_t t0 = l.toff[e / kPrepTile] + l.tpre[S.tp0 + c];
             for (uint32_t m = 0; m * T < cnt; ++m) {
                 Tile t;
                 t.key = (uint32_t)c;
@@ -151,106 +301,55 @@ __global__ __launch_bounds__(kPrepBlock) void k_ptilewrite(const PrepSeg *__rest
             const int cx = (int)(c % (uint64_t)S.g.nx);
             const int cy = (int)((c / (uint64_t)S.g.nx) % (uint64_t)S.g.ny);
             const int cz = (int)(c / ((uint64_t)S.g.nx * (uint64_t)S.g.ny));
+#pragma unroll 4
             for (int r = 0; r < S.nrows; ++r)
                 tot += row_count(S.rows[r], cx, cy, cz, S.g, S.cellstart);
         }
     }
-    // one atomic per wavefront and job: the lanes of a wave whose cells all
-    // belong to one job (the usual case) take their maximum first (a single
-    // counter line takes atomics one at a time)
-    const int j0 = __shfl(job, 0, 64);
-    const bool uniform = __all(job == j0) != 0;
-    if (uniform) {
-        for (int d = 32; d > 0; d >>= 1) {
-            const uint32_t o = (uint32_t)__shfl_xor((int)tot, d, 64);
-            tot = o > tot ? o : tot;
-        }
-        if ((threadIdx.x & 63) == 0 && tot > 0)
-            atomicMax(&js[j0].maxcand, tot);
-    } else if (tot > 0) {
-        atomicMax(&js[job].maxcand, tot);
+    // one atomic per wavefront (a block's cells belong to one job)
+    for (int d = 32; d > 0; d >>= 1) {
+        const uint32_t o = (uint32_t)__shfl_xor((int)tot, d, 64);
+        tot = o > tot ? o : tot;
     }
-}
-
-// Per job: its first center and tile in the run's lists and their counts
-// (a job's segments are consecutive).
-__global__ void k_pjobstat(const PrepSeg *__restrict__ segs, const int32_t *__restrict__ jseg,
-                           int njobs, const uint32_t *__restrict__ cpos,
-                           const uint32_t *__restrict__ toff, PrepJobStat *__restrict__ js)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= njobs)
-        return;
-    const int a = jseg[j], b = jseg[j + 1];
-    if (a == b) {
-        js[j].center0 = js[j].centers = js[j].tile0 = js[j].tiles = 0u;
-        return;
-    }
-    const PrepSeg &F = segs[a], &L = segs[b - 1];
-    js[j].center0 = cpos[F.ion0];
-    js[j].centers = cpos[L.ion0 + L.n] - cpos[F.ion0];
-    js[j].tile0 = toff[F.cell0];
-    js[j].tiles = toff[L.cell0 + L.nc] - toff[F.cell0];
-}
-
-__global__ void k_pclear(PrepJobStat *__restrict__ js, int njobs)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j < njobs)
-        js[j].maxcand = 0u;
-}
-
-unsigned grid_of(uint64_t n)
-{
-    uint64_t g = (n + kPrepBlock - 1) / kPrepBlock;
-    return (unsigned)(g ? g : 1);
+    if ((threadIdx.x & 63) == 0 && tot > 0)
+        atomicMax(&js[S.job].maxcand, tot);
 }
 
 } // namespace
 
-size_t prep_workspace_words(uint64_t E, uint64_t Ec)
+PrepWords prep_words(uint64_t E, uint64_t Ec, uint64_t nc)
 {
-    return scan_workspace_words(E > Ec ? E : Ec);
+    PrepWords w;
+    w.bits = E / 32;
+    w.wpos = E / 64;
+    w.boff = E / kPrepTile + 1;
+    w.tpre = nc;
+    w.toff = Ec / kPrepTile + 1;
+    return w;
 }
 
 hipError_t launch_prep(const PrepLaunch &p, hipStream_t s)
 {
     if (p.nseg <= 0 || p.njobs <= 0)
         return hipSuccess;
-    hipLaunchKernelGGL(k_pclear, dim3((p.njobs + 255) / 256), dim3(256), 0, s, p.js, p.njobs);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess)
+    const uint32_t nion = (uint32_t)(p.E / kPrepTile), ncell = (uint32_t)(p.Ec / kPrepTile);
+    hipError_t e;
+    hipLaunchKernelGGL(k_pflags, dim3(p.jblocks ? p.jblocks : 1), dim3(kPrepBlock), 0, s, p.segs, p.jseg, p.njobs,
+                       p.l, p.js);
+    if ((e = hipGetLastError()) != hipSuccess)
         return e;
-    if (p.E > 0) {
-        hipLaunchKernelGGL(k_pflags, dim3(grid_of(p.E)), dim3(kPrepBlock), 0, s, p.segs, p.nseg,
-                           p.E, p.flags);
-        if ((e = hipGetLastError()) != hipSuccess)
-            return e;
-    }
-    if ((e = scan_exclusive(p.flags, p.cpos, p.E, p.ws, s)) != hipSuccess)
+    hipLaunchKernelGGL(k_pscan, dim3(1), dim3(1024), 0, s, p.l.boff, nion);
+    if ((e = hipGetLastError()) != hipSuccess)
         return e;
-    if (p.E > 0) {
-        hipLaunchKernelGGL(k_pcompact, dim3(grid_of(p.E)), dim3(kPrepBlock), 0, s, p.segs, p.nseg,
-                           p.E, p.flags, p.cpos, p.centers);
-        if ((e = hipGetLastError()) != hipSuccess)
-            return e;
-    }
-    if (p.Ec > 0) {
-        hipLaunchKernelGGL(k_ptilecount, dim3(grid_of(p.Ec)), dim3(kPrepBlock), 0, s, p.segs,
-                           p.nseg, p.Ec, p.cpos, p.ntile);
-        if ((e = hipGetLastError()) != hipSuccess)
-            return e;
-    }
-    if ((e = scan_exclusive(p.ntile, p.toff, p.Ec, p.ws, s)) != hipSuccess)
+    hipLaunchKernelGGL(k_pcompact, dim3(nion + ncell ? nion + ncell : 1), dim3(kPrepBlock), 0, s, p.segs, p.nseg,
+                       nion, p.l, p.centers);
+    if ((e = hipGetLastError()) != hipSuccess)
         return e;
-    if (p.Ec > 0) {
-        hipLaunchKernelGGL(k_ptilewrite, dim3(grid_of(p.Ec)), dim3(kPrepBlock), 0, s, p.segs,
-                           p.nseg, p.Ec, p.cpos, p.toff, p.tiles, p.js);
-        if ((e = hipGetLastError()) != hipSuccess)
-            return e;
-    }
-    hipLaunchKernelGGL(k_pjobstat, dim3((p.njobs + 255) / 256), dim3(256), 0, s, p.segs, p.jseg,
-                       p.njobs, p.cpos, p.toff, p.js);
+    hipLaunchKernelGGL(k_pscan, dim3(1), dim3(1024), 0, s, p.l.toff, ncell);
+    if ((e = hipGetLastError()) != hipSuccess)
+        return e;
+    hipLaunchKernelGGL(k_ptilewrite, dim3(ncell ? ncell * kPrepItems : 1), dim3(kPrepBlock), 0, s,
+                       p.segs, p.nseg, p.jseg, p.njobs, p.l, p.tiles, p.js);
     return hipGetLastError();
 }
 
