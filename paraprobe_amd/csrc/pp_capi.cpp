@@ -2013,14 +2013,18 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
             }
         }
         {
-            // the RDF pair counts give the in-ball total when every ion type
-            // of the cloud is a neighbour type of the job
+            // the in-ball total needs no count of its own where the RDF pair
+            // counts give it, every ion type of the cloud being a neighbour
+            // type of the job, nor where there is none to give: a typed list
+            // holds the neighbour types only (pairs_inball is -1 below).  The
+            // count is a ballot and a 64-bit add per center and wavefront step.
             const JobPlan &p = runs[i].plan;
-            bool all_env = runs[i].cand == runs[i].cl;
+            const bool typed = runs[i].cand != runs[i].cl;
+            bool all_env = !typed;
             for (int t = 0; t < 256 && all_env; ++t)
                 if (clouds[i]->type_count[t] > 0 && p.envoff[t] < 0)
                     all_env = false;
-            runs[i].count_in = !(all_env && (p.families & (PP_FAM_RDF | PP_FAM_RIPK)));
+            runs[i].count_in = !typed && !(all_env && (p.families & (PP_FAM_RDF | PP_FAM_RIPK)));
         }
         runs[i].rows = make_rows(runs[i].cl->g.w, runs[i].cl->g.wyz, runs[i].plan.R);
         if ((int)runs[i].rows.size() > kMaxRows)
