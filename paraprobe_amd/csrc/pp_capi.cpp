@@ -73,12 +73,21 @@ struct CellList {
     size_t bytes = 0;
 };
 
+// A read-back of up to this size goes through a slot's pinned buffer (one copy
+// by the engine; pageable memory takes the runtime's own staging and waits).
+// A call's copies and fills were 10 and are 5: one upload for the tables and
+// segments, one for a launch group's descriptors and queue counters, one fill
+// for the counters and rerun marks, two read-backs (20,000 ions 283 and 211 us
+// per call, 1 million ions 282 and 206 us).
+constexpr size_t kPinBytes = size_t(256) << 10;
+
 struct Slot {
     hipStream_t stream = nullptr;
     DevBuf scratch;  // cell-list temporaries, job arenas
     DevBuf jobbuf;   // JobDev array + tile pointer table + tile offsets + queue
     DevBuf cnbuf;    // CNTNB counters
     DevBuf kbuf;     // k-th neighbour categories of one launch chunk
+    char *pin = nullptr;  // kPinBytes of pinned host memory: small read-backs
     hipEvent_t ev[6] = {};
     // event pairs around the query-kernel launches of the current call
     std::vector<hipEvent_t> qev;
@@ -221,6 +230,7 @@ pp_status slot_init(pp_ctx *c, Slot &s)
     PP_HIP(c, hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking));
     for (auto &e : s.ev)
         PP_HIP(c, hipEventCreate(&e));
+    PP_HIP(c, hipHostMalloc((void **)&s.pin, kPinBytes, hipHostMallocDefault));
     return PP_OK;
 }
 
@@ -235,6 +245,10 @@ void slot_free(Slot &s)
             b->p = nullptr;
             b->cap = 0;
         }
+    if (s.pin) {
+        (void)hipHostFree(s.pin);
+        s.pin = nullptr;
+    }
     for (auto &e : s.ev)
         if (e) {
             (void)hipEventDestroy(e);
@@ -887,9 +901,14 @@ void layout_prep(PrepArena &a, Carver &m, bool fixed)
     m.off = std::max(m.off, room.off);
     a.centers = m.take<uint32_t>(a.nion + 1);
     a.tiles = m.take<Tile>(a.nion + 1);  // at most one tile per center
+    a.js = m.take<PrepJobStat>((size_t)std::max(a.njobs, 1));
+}
+
+// The part of the arena that is uploaded (the run's tables follow it)
+void layout_prep_upload(PrepArena &a, Carver &m)
+{
     a.segs = m.take<PrepSeg>((size_t)std::max(a.nseg, 1));
     a.jseg = m.take<int32_t>((size_t)a.njobs + 1);
-    a.js = m.take<PrepJobStat>((size_t)std::max(a.njobs, 1));
 }
 
 // Bytes of one job's share of a run's scratch (admission control).
@@ -940,8 +959,11 @@ void stage_tables(const JobRun &r, uint32_t *h)
 // selected by the considered rule, or, for the full-range rerun, by the
 // job's rerun marks.  Reads back each job's center and tile counts and its
 // stencil candidate bound; the lists stay valid until the next prep_run.
+// tables: the run's tables, uploaded to tables_dev (behind the arena's segment
+// list) in the same copy, or null.
 pp_status prep_run(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std::vector<int> &ids,
-                   PrepArena &a, bool rerun)
+                   PrepArena &a, bool rerun, const std::vector<uint32_t> *tables,
+                   const uint32_t *tables_dev)
 {
     const int nj = (int)ids.size();
     if (nj == 0)
@@ -985,10 +1007,18 @@ pp_status prep_run(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std::ve
     if (E > a.E || Ec > a.Ec || nc > a.nc || (int)segs.size() > a.nseg || nj > a.njobs)
         return fail(c, PP_ERR_HIP, "internal: preparation larger than its arena");
     hipStream_t s = sl.stream;
-    if (!segs.empty())
-        PP_HIP(c, hipMemcpyAsync(a.segs, segs.data(), segs.size() * sizeof(PrepSeg),
-                                 hipMemcpyHostToDevice, s));
-    PP_HIP(c, hipMemcpyAsync(a.jseg, jseg.data(), jseg.size() * 4, hipMemcpyHostToDevice, s));
+    char *const up0 = (char *)a.segs;
+    std::vector<char> up(tables ? (size_t)((const char *)tables_dev - up0) + tables->size() * 4
+                                : (size_t)((const char *)a.jseg - up0) + jseg.size() * 4);
+    auto stage = [&](const void *dev, const void *src, size_t bytes) {
+        if (bytes)
+            std::memcpy(up.data() + ((const char *)dev - up0), src, bytes);
+    };
+    stage(a.segs, segs.data(), segs.size() * sizeof(PrepSeg));
+    stage(a.jseg, jseg.data(), jseg.size() * 4);
+    if (tables)
+        stage(tables_dev, tables->data(), tables->size() * 4);
+    PP_HIP(c, hipMemcpyAsync(up0, up.data(), up.size(), hipMemcpyHostToDevice, s));
     PrepLaunch L;
     L.segs = a.segs;
     L.nseg = (int)segs.size();
@@ -1002,12 +1032,15 @@ pp_status prep_run(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std::ve
     L.tiles = a.tiles;
     L.js = a.js;
     std::vector<PrepJobStat> js(nj);
+    const bool pin = nj * sizeof(PrepJobStat) <= kPinBytes;
     if (L.nseg > 0) {
         PP_HIP(c, launch_prep(L, s));
-        PP_HIP(c, hipMemcpyAsync(js.data(), a.js, nj * sizeof(PrepJobStat), hipMemcpyDeviceToHost,
-                                 s));
+        PP_HIP(c, hipMemcpyAsync(pin ? (void *)sl.pin : (void *)js.data(), a.js,
+                                 nj * sizeof(PrepJobStat), hipMemcpyDeviceToHost, s));
     }
-    PP_HIP(c, hipStreamSynchronize(s));  // segs and jseg are host memory of this frame
+    PP_HIP(c, hipStreamSynchronize(s));  // the upload is host memory of this frame
+    if (L.nseg > 0 && pin)
+        std::memcpy((void *)js.data(), sl.pin, nj * sizeof(PrepJobStat));
     for (int q = 0; q < nj; ++q) {
         JobRun &r = runs[ids[q]];
         r.h_counts[0] = js[q].centers;
@@ -1561,9 +1594,7 @@ void plan_chunks(const std::vector<const JobPlan *> &plans, const std::vector<ui
 // Host images of device tables handed to asynchronous copies; they must
 // outlive the launches that read them.
 struct Keep {
-    std::deque<std::vector<JobDev>> devs;
-    std::deque<std::vector<uint32_t>> words;
-    std::deque<std::vector<const Tile *>> tiles;
+    std::deque<std::vector<char>> bytes;
     bool graph = false;               // capture each group's launches into a graph
     hipStream_t stream = nullptr;     // the stream the graphs were launched on
     size_t ngraphs = 0;               // groups launched as graphs so far in this run
@@ -1658,14 +1689,14 @@ pp_status launch_group(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std
     uint32_t *d_off = jb.take<uint32_t>(nj + 1);
     uint32_t *d_uoff = jb.take<uint32_t>((size_t)(nj + 1) * nch);
     uint32_t *d_queue = jb.take<uint32_t>(kQueueWords);
-    keep.devs.emplace_back((size_t)nj * nch);
-    std::vector<JobDev> &hj = keep.devs.back();
-    keep.words.emplace_back((size_t)(nj + 1) * nch, 0u);
-    std::vector<uint32_t> &huoff = keep.words.back();
-    keep.words.push_back(tile_off);
-    const std::vector<uint32_t> &htoff = keep.words.back();
-    keep.tiles.emplace_back(nj);
-    std::vector<const Tile *> &ht = keep.tiles.back();
+    // the host image of the descriptors, uploaded in one copy; the first
+    // chunk's queue counters are its zeros
+    keep.bytes.emplace_back((size_t)((char *)(d_queue + kQueueWords) - (char *)d_jobs), 0);
+    std::vector<char> &image = keep.bytes.back();
+    auto host = [&](const void *dev) { return image.data() + ((const char *)dev - (char *)d_jobs); };
+    JobDev *const hj = (JobDev *)host(d_jobs);
+    uint32_t *const huoff = (uint32_t *)host(d_uoff);
+    std::memcpy(host(d_off), tile_off.data(), 4 * (size_t)(nj + 1));
     uint32_t tpu_max = 1;
     std::vector<uint32_t> tpus(nch);  // tiles per reduction unit, per chunk
     int red_lds = 0;
@@ -1715,13 +1746,8 @@ pp_status launch_group(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std
         huoff[k * (nj + 1) + nj] = units;
     }
     for (int q = 0; q < nj; ++q)
-        ht[q] = runs[ids[q]].tiles;
-    PP_HIP(c, hipMemcpyAsync(d_jobs, hj.data(), sizeof(JobDev) * hj.size(), hipMemcpyHostToDevice,
-                             sl.stream));
-    PP_HIP(c, hipMemcpyAsync(d_tiles, ht.data(), sizeof(Tile *) * nj, hipMemcpyHostToDevice,
-                             sl.stream));
-    PP_HIP(c, hipMemcpyAsync(d_off, htoff.data(), 4 * (nj + 1), hipMemcpyHostToDevice, sl.stream));
-    PP_HIP(c, hipMemcpyAsync(d_uoff, huoff.data(), 4 * huoff.size(), hipMemcpyHostToDevice,
+        ((const Tile **)host(d_tiles))[q] = runs[ids[q]].tiles;
+    PP_HIP(c, hipMemcpyAsync(d_jobs, image.data(), image.size(), hipMemcpyHostToDevice,
                              sl.stream));
     int nb = 0;
     PP_HIP(c, query_max_blocks_per_cu(T, c16, mode, lds, &nb));
@@ -1733,7 +1759,7 @@ pp_status launch_group(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std
                      "maxC=%d maxE=%d maxTrg=%d kmax=%d rows=%d HK=%d\n",
                      mode, T, c16, lds, nb, nj, total, nch, maxC, maxE, maxTrg, maxK, maxRows,
                      maxHK);
-    const bool capture = keep.graph && nch > 0;  // (no empty graphs)
+    const bool capture = keep.graph && total > 0;  // (no empty graphs)
     if (capture)
         PP_HIP(c, hipStreamBeginCapture(sl.stream, hipStreamCaptureModeRelaxed));
     hipError_t le = hipSuccess;
@@ -1747,6 +1773,7 @@ pp_status launch_group(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std
         ql.first_tile = ch.g0;
         ql.end_tile = ch.g1;
         ql.queue = d_queue;
+        ql.queue_zero = k == 0;
         ql.T = T;
         ql.c16 = c16;
         ql.mode = mode;
@@ -2069,18 +2096,31 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
         layout_tables(runs[i]);
         tables_words += runs[i].tables_words;
     }
+    // a hybrid job with a kNN range short of Rmax
+    auto may_rerun = [](const JobRun &r) { return r.plan.mode == 2 && r.plan.trunc_any; };
+    uint32_t *tables_dev = nullptr;
+    char *clear1 = nullptr;
     auto carve = [&](Carver &m, char *&out0, char *&out1) {
         out0 = m.base ? m.base + ((m.off + 255) & ~(size_t)255) : nullptr;
         for (int i = 0; i < njobs; ++i)
             layout_outputs(runs[i], m);
         out1 = m.base ? m.base + m.off : nullptr;
-        uint32_t *tab = m.take<uint32_t>(tables_words);
+        // the marks of the jobs that may rerun first: cleared with the counters
+        clear1 = out1;
+        for (bool may : {true, false})
+            for (int i = 0; i < njobs; ++i)
+                if (may_rerun(runs[i]) == may) {
+                    runs[i].flags = m.take<uint32_t>(runs[i].cloud->n + 1);
+                    if (may)
+                        clear1 = m.base ? m.base + m.off : nullptr;
+                }
+        layout_prep_upload(pa, m);
+        tables_dev = m.take<uint32_t>(tables_words);
+        uint32_t *tab = tables_dev;
         for (int i = 0; i < njobs; ++i) {
             runs[i].tables = tab;
             tab = tab ? tab + runs[i].tables_words : nullptr;
         }
-        for (int i = 0; i < njobs; ++i)
-            runs[i].flags = m.take<uint32_t>(runs[i].cloud->n + 1);
         layout_prep(pa, m, sl.fixed != nullptr);
     };
     char *out0 = nullptr, *out1 = nullptr;
@@ -2099,30 +2139,30 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
             stage_tables(runs[i], h.data() + o);
             o += runs[i].tables_words;
         }
-        if (tables_words)
-            PP_HIP(c, hipMemcpyAsync(runs[0].tables, h.data(), tables_words * 4,
-                                     hipMemcpyHostToDevice, sl.stream));
-        PP_HIP(c, hipMemsetAsync(out0, 0, out_bytes, sl.stream));
+        PP_HIP(c, hipMemsetAsync(out0, 0, (size_t)(clear1 - out0), sl.stream));
         std::vector<int> all(njobs);
         for (int i = 0; i < njobs; ++i)
             all[i] = i;
-        st = prep_run(c, sl, runs, all, pa, false);  // synchronises: h may go
+        st = prep_run(c, sl, runs, all, pa, false, &h, tables_dev);
         if (st != PP_OK)
             return st;
     }
     PP_HIP(c, hipEventRecord(sl.ev[2], sl.stream));
     size_t cn_words = 0;
+    bool cntnb = false;
     {
         // CNTNB counters: no neighbour count exceeds the largest stencil candidate count
         for (int i = 0; i < njobs; ++i) {
             JobRun &r = runs[i];
             r.cn_cap = (r.plan.families & PP_FAM_CNTNB) ? (int)r.h_counts[2] + 1 : 1;
+            cntnb = cntnb || (r.plan.families & PP_FAM_CNTNB);
             cn_words += ((size_t)std::max(r.plan.ntasks, 1) * (size_t)r.cn_cap + 63) & ~(size_t)63;
         }
         st = ensure(c, sl, sl.cnbuf, cn_words * 4 + 256);
         if (st != PP_OK)
             return st;
-        PP_HIP(c, hipMemsetAsync(sl.cnbuf.p, 0, cn_words * 4, sl.stream));
+        if (cntnb)
+            PP_HIP(c, hipMemsetAsync(sl.cnbuf.p, 0, cn_words * 4, sl.stream));
         size_t o = 0;
         for (int i = 0; i < njobs; ++i) {
             JobRun &r = runs[i];
@@ -2191,23 +2231,14 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
     {
         std::vector<int> ids, modes;
         std::vector<JobDev> devs;
-        // the rerun marks of the jobs that may rerun, cleared by one memset
-        // over their span (the jobs' marks are carved one after another)
-        char *mk0 = nullptr, *mk1 = nullptr;
         for (int i = 0; i < njobs; ++i) {
             JobRun &r = runs[i];
             ids.push_back(i);
             devs.push_back(r.dev);
             modes.push_back(r.plan.mode);
-            if (r.plan.mode == 2 && r.plan.trunc_any) {
-                char *b0 = (char *)r.flags, *b1 = (char *)(r.flags + r.cloud->n);
-                mk0 = mk0 && mk0 < b0 ? mk0 : b0;
-                mk1 = mk1 && mk1 > b1 ? mk1 : b1;
+            if (may_rerun(r))
                 hy.push_back(i);
-            }
         }
-        if (mk0 && mk1 > mk0)
-            PP_HIP(c, hipMemsetAsync(mk0, 0, (size_t)(mk1 - mk0), sl.stream));
         if (order) {
             turn.take();
             if (order->armed)
@@ -2237,7 +2268,7 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
                            c->lds_per_block)
                     r.T_req /= 2;
             }
-            st = prep_run(c, sl, runs, hy, pa, true);
+            st = prep_run(c, sl, runs, hy, pa, true, nullptr, nullptr);
             if (st != PP_OK)
                 return st;
             std::vector<int> ids1, modes1;
@@ -2272,12 +2303,12 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
         }
         PP_HIP(c, hipEventRecord(sl.ev[4], sl.stream));
         // read back (the counters of every job in one copy)
-        std::vector<char> hout(out_bytes);
-        std::vector<uint32_t> hcn(cn_words);
+        std::vector<char> hbuf(out_bytes <= kPinBytes ? 0 : out_bytes);
+        char *const hout = hbuf.empty() ? sl.pin : hbuf.data();
+        std::vector<uint32_t> hcn(cntnb ? cn_words : 0);
         if (out_bytes)
-            PP_HIP(c, hipMemcpyAsync(hout.data(), out0, out_bytes, hipMemcpyDeviceToHost,
-                                     sl.stream));
-        if (cn_words)
+            PP_HIP(c, hipMemcpyAsync(hout, out0, out_bytes, hipMemcpyDeviceToHost, sl.stream));
+        if (cntnb && cn_words)
             PP_HIP(c, hipMemcpyAsync(hcn.data(), sl.cnbuf.p, cn_words * 4, hipMemcpyDeviceToHost,
                                      sl.stream));
         if (order) {
@@ -2294,7 +2325,7 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
             JobRun &r = runs[i];
             const JobPlan &p = r.plan;
             Back &b = back[i];
-            auto host = [&](const void *dev) { return hout.data() + ((const char *)dev - out0); };
+            auto host = [&](const void *dev) { return hout + ((const char *)dev - out0); };
             b.P.resize((size_t)std::max(p.ntrg * p.E * p.C, 1));
             std::memcpy(b.P.data(), host(r.P), b.P.size() * 8);
             std::memcpy(b.stats, host(r.stats), sizeof(b.stats));

@@ -1745,12 +1745,14 @@ __global__ __launch_bounds__(64) void k_queue_clear(uint32_t *__restrict__ q)
 hipError_t launch_query(const QueryLaunch &q, hipStream_t s)
 {
     const int T = q.T, c16 = q.c16, mode = q.mode;
-    hipLaunchKernelGGL(k_queue_clear, dim3(1), dim3(64), 0, s, q.queue);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess)
-        return e;
     if (q.end_tile <= q.first_tile)
         return hipSuccess;
+    if (!q.queue_zero) {
+        hipLaunchKernelGGL(k_queue_clear, dim3(1), dim3(64), 0, s, q.queue);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess)
+            return e;
+    }
     PP_DISPATCH(launch_query_t, q, s);
 }
 

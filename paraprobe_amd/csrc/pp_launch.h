@@ -124,7 +124,8 @@ struct QueryLaunch {
     const Tile *const *tiles;  // device [njobs] per-job tile arrays
     uint32_t first_tile;       // global tile range [first_tile, end_tile) of this launch
     uint32_t end_tile;
-    uint32_t *queue;           // device counters (kQueueWords), zeroed by the launcher
+    uint32_t *queue;           // device counters (kQueueWords)
+    int queue_zero;            // 1: they are zero already, 0: the launcher clears them
     uint32_t grab;             // tiles handed out per queue atomic
     int T;                     // centers per tile
     int c16;                   // 16-bit per-center counters
