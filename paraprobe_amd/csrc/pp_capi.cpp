@@ -1749,8 +1749,32 @@ pp_status launch_group(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std
         ((const Tile **)host(d_tiles))[q] = runs[ids[q]].tiles;
     PP_HIP(c, hipMemcpyAsync(d_jobs, image.data(), image.size(), hipMemcpyHostToDevice,
                              sl.stream));
+    // the k-th neighbour extraction's table of tasks and, beyond what the
+    // stencil rows' words hold, its entries get LDS words of their own where
+    // that leaves as many workgroups on a CU
+    int taskw = 0, entw = 0;
+    if (mode != 0) {
+        int maxL = 0, keff = 0;
+        for (const JobPlan *p : plans) {
+            maxL = std::max(maxL, p->lmax);
+            keff = std::max(keff, p->kmax);
+        }
+        auto wgs = [&](size_t l) { return (size_t(160) << 10) / ((l + 511) / 512 * 512); };
+        auto room = [&](size_t words) {
+            const size_t l = lds + 4 * words;
+            return l <= c->lds_per_block && wgs(l) == wgs(lds);
+        };
+        for (int n : {std::min(maxL, 64), std::min(maxL, 8)})
+            if (!taskw && room(4 * (size_t)n))
+                taskw = 4 * n;
+        const int need = ((c16 ? 2 : 1) * std::max(keff, 1) + 1) / 2;
+        if (need > query_row_words(maxRows, mode) / kWaves &&
+            room((size_t)taskw + (size_t)kWaves * (size_t)need))
+            entw = need;
+    }
+    const size_t lds_all = lds + 4 * ((size_t)taskw + (size_t)kWaves * (size_t)entw);
     int nb = 0;
-    PP_HIP(c, query_max_blocks_per_cu(T, c16, mode, lds, &nb));
+    PP_HIP(c, query_max_blocks_per_cu(T, c16, mode, lds_all, &nb));
     if (nb < 1)
         nb = 1;
     if (std::getenv("PP_TRACE_LAUNCH"))
@@ -1785,6 +1809,8 @@ pp_status launch_group(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std
         ql.maxRows = maxRows;
         ql.maxHK = maxHK;
         ql.maxP = maxP;
+        ql.taskw = taskw;
+        ql.entw = entw;
         const uint32_t want = (uint32_t)c->cu_count * (uint32_t)nb;
         ql.grid = (int)std::max<uint32_t>(
             1u, std::min<uint32_t>(want, std::max<uint32_t>(ch.g1 - ch.g0, 1u)));

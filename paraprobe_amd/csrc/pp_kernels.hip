@@ -571,20 +571,22 @@ __host__ __device__ inline Lay make_layout(int T, int c16, int mode, int maxC, i
     o += al4(2 * maxRows);
     L.rowpre = o;  // per row its first index in the rows' concatenation
     o += al4(maxRows + 1);
-    // after the main loop these words hold the tile's tasks and, at their
-    // end, per wavefront the k window of the k-th category extraction (uint16)
+    // after the main loop these words hold the entries of the k-th category
+    // extraction or, for k beyond what they hold, at their end per wavefront
+    // its k window (both uint16)
     if (mode && o < L.rows + kWinWords + 24)
         o = L.rows + kWinWords + 24;
     L.win = mode ? o - kWinWords : o;
     L.cen = o;
     o += 4 * T;
     L.meta = o;
-    o += al4(2 * T);
+    o += al4(T);
     L.P = o;
     o += al4(maxP);  // pair counts of one center type (tiles hold one type)
     L.H = o;
     const int hc = c16 ? (T + 1) / 2 : T;
-    o += mode == 1 ? al4(hc * maxE * maxC) : mode == 2 ? al4(hc * maxHK) : 0;
+    // (and 4 words behind them: the extraction reads 4 categories at a time)
+    o += mode == 1 ? al4(hc * maxE * maxC) + 4 : mode == 2 ? al4(hc * maxHK) + 4 : 0;
     L.total = o;
     return L;
 }
@@ -598,6 +600,12 @@ size_t query_lds_bytes(int T, int c16, int mode, int maxC, int maxE, int maxTrg,
            4u;
 }
 
+int query_row_words(int maxRows, int mode)
+{
+    const Lay L = make_layout(8, 1, mode, 1, 1, 1, 0, maxRows, 1, 1, 1);
+    return L.cen - L.rows;
+}
+
 struct QArgs {
     const JobDev *jobs;
     const uint32_t *tile_off;
@@ -608,6 +616,7 @@ struct QArgs {
     int njobs;
     int maxC, maxE, maxTrg, maxKmax, maxRows, maxHK, maxP;
     int ntypes;  // type ids of the launch's candidates are below this
+    int taskw, entw;  // QueryLaunch
 };
 
 __device__ inline int find_job(const uint32_t *__restrict__ off, int njobs, uint32_t g)
@@ -744,7 +753,7 @@ __device__ inline int category_of(float d2, float isc, float ioff1, float ioffa,
 // range only (see JobDev::HK); centers whose kNN range holds too few
 // neighbours are flagged for a MODE 1 rerun.
 // Resident waves per SIMD asked of the compiler for 8-center tiles: 7 in the
-// pair-count mode (72 VGPRs, no spills), 6 in the hybrid mode (7 fits in 72
+// pair-count mode (71 VGPRs, no spills), 6 in the hybrid mode (77; 7 fits in 72
 // VGPRs with spills in the per-tile code: 0.3 % faster on the 20M-ion job,
 // 13 % slower on the 100M-ion one, whose tiles are cheaper).
 template <int T, bool C16, int MODE>
@@ -766,11 +775,15 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
     uint32_t *s_rows = lds + L.rows;
     uint32_t *s_rowpre = lds + L.rowpre;
     float4 *s_cen = (float4 *)(lds + L.cen);
-    uint32_t *s_meta = lds + L.meta;  // [2c] tc | es << 8, [2c+1] unused
+    uint32_t *s_meta = lds + L.meta;  // tc | es << 8
     uint32_t *s_P = lds + L.P;
     uint32_t *s_H = lds + L.H;
+    // per task of the center type: its id, its neighbour types, its kNN-range
+    // categories and, when it has one neighbour type, that type's row in a
+    // center's histogram (else -1)
+    uint32_t *s_task = lds + L.total;
 
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
+    int tid = threadIdx.x;
     int cur = -1;
     // tile queues (one counter per XCD); thread 0 keeps the grab state
     const uint32_t myx = xcc_id() & (uint32_t)(kXcds - 1);
@@ -781,6 +794,11 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
     unsigned long long pending = 0;  // pairs accumulated in s_P since its last flush
 
     for (;;) {
+        // (opaque per tile: what a tile's code derives from the thread's
+        // number is computed where it is used, not kept in registers, or
+        // spilled, across the main loop)
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & (kWave - 1), wid = (int)rfl((uint32_t)tid / kWave);
         __syncthreads();
         if (tid == 0)
             s_g = next_tile(a, myx, qx, gnext, left);
@@ -859,6 +877,20 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                     for (int i = tid; i <= J.kmax; i += kBlock)
                         s_kidx[i] = J.kidx_of_k ? J.kidx_of_k[i] : -1;
             }
+            if (PC || HY) {
+                const int Ls = min((int)J.trg_ntask[ts], a.taskw / 4);
+                for (int l = tid; l < Ls; l += kBlock) {
+                    const uint32_t tk = J.trg_tasks[ts * J.lmax + l];
+                    const uint32_t envset = J.task_env[tk];
+                    s_task[4 * l] = tk;
+                    s_task[4 * l + 1] = envset;
+                    s_task[4 * l + 2] = HY ? J.task_ck[tk] : (uint32_t)J.C;
+                    const int e = envset ? __builtin_ctz(envset) : 0;
+                    s_task[4 * l + 3] = __builtin_popcount(envset) != 1 ? ~0u
+                                        : PC                            ? (uint32_t)(e * J.C)
+                                                                        : (uint32_t)J.ckoff[e];
+                }
+            }
             const int n =
                 (J.E + (MODE == 0 && ts == J.sym_slot ? __builtin_popcount(J.sym_minor) : 0)) * J.C;
             for (int i = tid; i < n; i += kBlock)
@@ -901,7 +933,7 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                 if (eo >= 0)
                     es = (uint32_t)__builtin_rintf((float)eo * __builtin_amdgcn_rcpf((float)C));
             }
-            s_meta[2 * tid] = (uint32_t)ts | (es << 8);
+            s_meta[tid] = (uint32_t)ts | (es << 8);
             s_cen[tid] = make_float4(px, py, pz, 0.f);
         }
         __syncthreads();
@@ -1422,7 +1454,7 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
         if (!PC) {
             // remove the self pair (d = 0) each center added to its own type
             if (tid < cnt) {
-                const uint32_t m = s_meta[2 * tid];
+                const uint32_t m = s_meta[tid];
                 const uint32_t es = (m >> 8) & 0xFFu;
                 if (es != 0xFFu)
                     __hip_atomic_fetch_add(&s_P[es * C + J.cat0], 0xFFFFFFFFu,
@@ -1438,28 +1470,13 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
         // first (in a 16-bit half the count holds that pair, so nothing
         // borrows from the other half)
         if (tid < cnt) {
-            const uint32_t es = (s_meta[2 * tid] >> 8) & 0xFFu;
+            const uint32_t es = (s_meta[tid] >> 8) & 0xFFu;
             if (es != 0xFFu) {
                 const int h0 = (C16 ? (tid >> 1) : tid) * (PC ? EC : HK) +
                                (PC ? (int)es * C : s_ckoff[es]) + cat0;
                 __hip_atomic_fetch_add(&s_H[h0], (C16 && (tid & 1)) ? 0xFFFF0000u : 0xFFFFFFFFu,
                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
-        }
-        // the tasks of the tile's center type (every center of a tile has
-        // it): per task l its id, env set and kNN-range categories, read once
-        // here rather than by each center's wave in series, into the stencil
-        // rows' words (free until the next tile) as far as they hold them
-        const int Lt = (int)J.trg_ntask[ts];
-        // (the rows' starts and prefix hold L.win - L.rows words before the
-        // extraction's windows)
-        const int Ls = Lt < (L.win - L.rows) / 3 ? Lt : (L.win - L.rows) / 3;
-        uint32_t *s_task = s_rows;  // (the main loop's closing barrier freed them)
-        for (int l = tid; l < Ls; l += kBlock) {
-            const uint32_t tk = J.trg_tasks[ts * J.lmax + l];
-            s_task[3 * l] = tk;
-            s_task[3 * l + 1] = J.task_env[tk];
-            s_task[3 * l + 2] = HY ? J.task_ck[tk] : (uint32_t)C;
         }
         __syncthreads();
         if (PC && (J.families & (FAM_RDF | FAM_RIPK))) {
@@ -1473,11 +1490,19 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
             }
         }
         if (want_k || want_1 || want_cn) {
+            // (the thread's numbers behind an opaque value: what the code
+            // below derives from them is computed here, not kept in registers
+            // through the main loop)
+            uint32_t xt = (uint32_t)tid;
+            asm volatile("" : "+v"(xt));
+            const int lane = (int)(xt & (kWave - 1)), wid = (int)rfl(xt / kWave);
             const int kmax = want_k ? J.kmax : 0;
             const bool kdense = J.k_dense != 0;
             const uint32_t need = want_k ? (uint32_t)kmax : 1u;
             const int lmax = J.lmax;
             // this tile's block of k-th neighbour rows in the chunk buffer
+            const int Lt = (int)rfl((uint32_t)J.trg_ntask[ts]);
+            const int Ls = min(Lt, a.taskw / 4);
             const uint64_t tl = (uint64_t)(g - a.tile_off[job] - J.tile_base);
             const uint64_t TR = (uint64_t)T * (uint64_t)lmax;
             // stored through the global address space: a flat store counts
@@ -1492,7 +1517,164 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
             // test is skipped, not masked, when the job has no 1NN
             int w1 = (int)rfl(want_1 ? 1u : 0u);
             asm volatile("" : "+s"(w1));
-            for (int c = wid; c < cnt; c += kWaves) {
+            // the rerun settles this center: every plane of its rows (some
+            // already written) is emptied for the reduction
+            auto empty_rows = [&](int c) {
+                if (lane == 0)
+                    J.unres[J.centers[t_first + c]] = 1u;
+                const int np = J.nplanes;
+                if (kb)
+                    for (int i = lane; i < np * Lt; i += kWave) {
+                        const int pl = i / Lt, l = i - pl * Lt;
+                        kb[(uint32_t)pl * (uint32_t)TR + (uint32_t)(c * lmax + l)] = kKbEmpty;
+                    }
+            };
+            // Two centers (one with 32-bit counters) of a wavefront at a time,
+            // as the histograms hold them: their counts share a word, so one
+            // scan of the words gives both centers' neighbours before each
+            // category.  Per task a lane takes 4 categories of a step; a lane
+            // that holds neighbours leaves its group's number at its first
+            // one's k in the entries (center, k).  Then the entries are
+            // settled 64 at a time (lane = entry): a running maximum carries
+            // each mark to the k after it, and the group's 4 words, read
+            // again, give the category.  The kernel's
+            // times with one center, 2 categories a lane and a mark per
+            // category, as below, and now: 100 million ions, k to 20, 394 and
+            // 334 ms (293 ms without any extraction); 20 million, k to 100,
+            // 153 and 147 ms (136).
+            constexpr int UC = C16 ? 2 : 1;
+            const int keff = want_k ? kmax : 1;  // entries per task and center
+            const int ne = UC * keff;
+            // a wave's entries: in words of their own, or in the stencil
+            // rows' (free until the next tile) as far as these hold them
+            const int ewords =
+                a.entw > 0 ? a.entw : (L.cen - L.rows) / kWaves;
+            uint16_t *ent =
+                (uint16_t *)(a.entw > 0 ? s_task + a.taskw : s_rows) + 2 * ewords * wid;
+            const bool fits = ne <= 2 * ewords;
+            const int nunit =
+                (want_k || want_1) && kb && fits ? (cnt + UC - 1) / UC : 0;
+            for (int u = wid; u < nunit; u += kWaves) {
+                const int hoff = u * (PC ? EC : HK);
+                const int nh = cnt - u * UC < UC ? 1 : UC;  // centers of this unit
+                // centers whose range of a task holds fewer than it needs
+                uint32_t shortm = 0u;
+                for (int l = 0; l < Lt && shortm != (1u << nh) - 1u; ++l) {
+                    uint32_t envset, ckw;
+                    int off = -1;  // the one type's row
+                    if (l < Ls) {
+                        envset = rfl(s_task[4 * l + 1]);
+                        ckw = rfl(s_task[4 * l + 2]);
+                        off = (int)rfl(s_task[4 * l + 3]);
+                    } else {
+                        const uint32_t tk = J.trg_tasks[ts * lmax + l];
+                        envset = rfl(J.task_env[tk]);
+                        ckw = rfl(HY ? J.task_ck[tk] : (uint32_t)C);
+                    }
+                    const int ck = HY ? (int)(ckw & 0x7FFFFFFFu) : C;
+                    // the words of categories ca .. ca + 3, summed over the
+                    // task's types
+                    auto load4 = [&](int ca, uint32_t v[4]) __attribute__((always_inline)) {
+                        if (off >= 0) {
+                            const uint32_t *h = s_H + hoff + off + ca;
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                v[j] = h[j];
+                        } else {
+                            v[0] = v[1] = v[2] = v[3] = 0u;
+                            for (uint32_t w = envset; w; w &= w - 1u) {
+                                const int e = __builtin_ctz(w);
+                                const uint32_t *h = s_H + hoff + (PC ? e * C : s_ckoff[e]) + ca;
+#pragma unroll
+                                for (int j = 0; j < 4; ++j)
+                                    v[j] += h[j];
+                            }
+                        }
+                    };
+                    for (int i = lane; i < ne; i += kWave)
+                        ent[i] = 0u;
+                    uint32_t carry = 0u, tot0 = 0u, tot1 = need;
+                    for (int cb = 0; cb < ck; cb += 4 * kWave) {
+                        const int ca = cb + 4 * lane;
+                        uint32_t v[4] = {0u, 0u, 0u, 0u};
+                        if (ca < ck)
+                            load4(ca, v);
+                        if (cb + 4 * kWave > ck) {
+                            v[1] = ca + 1 < ck ? v[1] : 0u;
+                            v[2] = ca + 2 < ck ? v[2] : 0u;
+                            v[3] = ca + 3 < ck ? v[3] : 0u;
+                        }
+                        const uint32_t sum = (v[0] + v[1]) + (v[2] + v[3]);
+                        const uint32_t incl = wave_incl_scan(sum, lane);
+                        const uint32_t excl = carry + incl - sum;
+#pragma unroll
+                        for (int h = 0; h < UC; ++h) {
+                            const uint32_t sv = C16 ? (h ? sum >> 16 : sum & 0xFFFFu) : sum;
+                            const uint32_t ev = C16 ? (h ? excl >> 16 : excl & 0xFFFFu) : excl;
+                            if (sv != 0u && ev < (uint32_t)keff)
+                                ent[h * keff + (int)ev] = (uint16_t)((ca >> 2) + 1);
+                        }
+                        carry += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+                        tot0 = C16 ? carry & 0xFFFFu : carry;
+                        if (nh == 2)
+                            tot1 = carry >> 16;
+                        if (tot0 >= need && tot1 >= need)
+                            break;
+                    }
+                    // a task whose kNN range is short of the full range must
+                    // hold its k neighbours there, else the center is rerun
+                    // over the full range (its rows here are then marked
+                    // empty)
+                    if (HY && (ckw >> 31))
+                        shortm |= (tot0 < need ? 1u : 0u) | (tot1 < need ? 2u : 0u);
+                    uint32_t last = 0u;
+                    for (int i0 = 0; i0 < ne; i0 += kWave) {
+                        const int i = i0 + lane;
+                        const uint32_t raw = i < ne ? ent[i] : 0u;
+                        // (the mark's position above its group, so that the
+                        // later mark is the larger)
+                        const uint32_t m = __builtin_elementwise_max(
+                            wave_max_scan(raw ? ((uint32_t)(i + 1) << 16) | raw : 0u), last);
+                        last = (uint32_t)__builtin_amdgcn_readlane((int)m, kWave - 1);
+                        const int h = C16 && i >= keff ? 1 : 0;
+                        const int k1 = h ? i - keff : i;  // k - 1
+                        const int pos = (int)(m >> 16) - 1;
+                        const bool have = pos >= i - k1;  // a mark of this center
+                        // neighbours of the mark's group up to this k
+                        const uint32_t rem = (uint32_t)(i + 1 - pos);
+                        const int ca = have ? 4 * ((int)(m & 0xFFFFu) - 1) : 0;
+                        uint32_t v[4];
+                        load4(ca, v);
+                        const int sh = 16 * h;
+                        uint32_t run = 0u;
+                        int cat = ca - 1;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            cat += rem > run ? 1 : 0;
+                            run += C16 ? (v[j] >> sh) & 0xFFFFu : v[j];
+                        }
+                        // fewer than k env neighbours: R + EPSILON, i.e. the
+                        // sentinel category (S.cpp:4093-4095, 4035-4036)
+                        const uint16_t val =
+                            have && rem <= run && cat < ck ? (uint16_t)cat : sentinel;
+                        if (i < ne && h < nh) {
+                            const uint32_t row = (uint32_t)((u * UC + h) * lmax + l);
+                            if (want_k) {
+                                const int kid = kdense ? k1 : s_kidx[k1 + 1];
+                                if (kid >= 0)
+                                    kb[(uint32_t)kid * (uint32_t)TR + row] = val;
+                            }
+                            if (w1 != 0 && k1 == 0)
+                                kb[p1nn + row] = val;
+                        }
+                    }
+                }
+                for (int h = 0; h < nh; ++h)
+                    if (HY && ((shortm >> h) & 1u))
+                        empty_rows(u * UC + h);
+            }
+            // k beyond what the entries hold
+            for (int c = wid; c < cnt && !fits; c += kWaves) {
                 const int hoff = (C16 ? (c >> 1) : c) * (PC ? EC : HK);
                 const int sh = (C16 && (c & 1)) ? 16 : 0;
                 // count of env slot e, category cat in this center's histogram
@@ -1502,18 +1684,17 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                         s_H[hoff + (PC ? e * C : (int)rfl((uint32_t)s_ckoff[e])) + cat];
                     return C16 ? ((w >> sh) & 0xFFFFu) : w;
                 };
-                const int L = Lt;
                 // a task whose kNN range is short of the full range must hold
                 // its k neighbours there, else the center is rerun over the
                 // full range (its rows here are then marked empty)
                 bool short_range = false;
-                for (int l = 0; l < L; ++l) {
+                for (int l = 0; l < Lt; ++l) {
                     const bool st = l < Ls;
-                    const int tk = (int)rfl(st ? s_task[3 * l] : J.trg_tasks[ts * lmax + l]);
+                    const int tk = (int)rfl(st ? s_task[4 * l] : J.trg_tasks[ts * lmax + l]);
                     const int row = c * lmax + l;
-                    const uint32_t envset = rfl(st ? s_task[3 * l + 1] : J.task_env[tk]);
+                    const uint32_t envset = rfl(st ? s_task[4 * l + 1] : J.task_env[tk]);
                     const uint32_t ckw =
-                        rfl(st ? s_task[3 * l + 2] : (HY ? J.task_ck[tk] : (uint32_t)C));
+                        rfl(st ? s_task[4 * l + 2] : (HY ? J.task_ck[tk] : (uint32_t)C));
                     const int ck = HY ? (int)(ckw & 0x7FFFFFFFu) : C;
                     if ((want_k || want_1) && kb) {
                         // categories of the k-th nearest neighbours: a prefix
@@ -1630,13 +1811,26 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                             while (kw < (uint32_t)kmax)
                                 flush(carry);
                     }
-                    if (PC && want_cn) {
+                }
+                if (HY && short_range)
+                    empty_rows(c);
+            }
+            if (PC && want_cn)
+                for (int c = wid; c < cnt; c += kWaves) {
+                    const int hoff = (C16 ? (c >> 1) : c) * EC;
+                    const int sh = (C16 && (c & 1)) ? 16 : 0;
+                    for (int l = 0; l < Lt; ++l) {
+                        const bool st = l < Ls;
+                        const int tk = (int)rfl(st ? s_task[4 * l] : J.trg_tasks[ts * lmax + l]);
+                        const uint32_t envset = rfl(st ? s_task[4 * l + 1] : J.task_env[tk]);
                         for (int e = 0; e < E; ++e) {
                             if (!((envset >> e) & 1u))
                                 continue;
                             uint32_t tot = 0;
-                            for (int cat = lane; cat < C; cat += kWave)
-                                tot += hv(e, cat);
+                            for (int cat = lane; cat < C; cat += kWave) {
+                                const uint32_t w = s_H[hoff + e * C + cat];
+                                tot += C16 ? ((w >> sh) & 0xFFFFu) : w;
+                            }
                             for (int d = kWave / 2; d > 0; d >>= 1)
                                 tot += __shfl_xor(tot, d, kWave);
                             if (lane == 0) {
@@ -1648,20 +1842,6 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                         }
                     }
                 }
-                if (HY && short_range) {
-                    // the rerun settles this center: every plane of its rows
-                    // (some already written) is emptied for the reduction
-                    if (lane == 0)
-                        J.unres[J.centers[t_first + c]] = 1u;
-                    if (kb) {
-                        const int np = J.nplanes;
-                        for (int i = lane; i < np * L; i += kWave) {
-                            const int pl = i / L, l = i - pl * L;
-                            kb[(uint32_t)pl * (uint32_t)TR + (uint32_t)(c * lmax + l)] = kKbEmpty;
-                        }
-                    }
-                }
-            }
         }
     }
 }
@@ -1669,7 +1849,7 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
 template <int T, bool C16, int MODE>
 static hipError_t launch_query_t(const QueryLaunch &q, hipStream_t s)
 {
-    const size_t lds = query_lds_bytes(T, C16, MODE, q.maxC, q.maxE, q.maxTrg, q.maxKmax,
+    const size_t base = query_lds_bytes(T, C16, MODE, q.maxC, q.maxE, q.maxTrg, q.maxKmax,
                                        q.maxRows, q.maxHK, q.maxP, q.ntypes);
     QArgs a;
     a.jobs = q.jobs;
@@ -1688,6 +1868,9 @@ static hipError_t launch_query_t(const QueryLaunch &q, hipStream_t s)
     a.maxRows = q.maxRows;
     a.maxHK = q.maxHK;
     a.maxP = q.maxP;
+    a.taskw = q.taskw;
+    a.entw = q.entw;
+    const size_t lds = base + 4 * ((size_t)q.taskw + (size_t)kWaves * (size_t)q.entw);
     hipError_t e = hipFuncSetAttribute((const void *)k_query<T, C16, MODE>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess)

@@ -133,11 +133,15 @@ struct QueryLaunch {
     // maxKmax: the largest kmax of the jobs whose k are not 1..kmax (0: none)
     int maxC, maxE, maxTrg, maxKmax, maxRows, maxHK;
     int maxP;                  // LDS words of a tile's pair-count rows (JobDev::xrow's included)
+    int taskw, entw;           // further LDS words: of the tasks' table (4 a task), and a wave's
+                               // of the k-th neighbour entries (0: in the stencil rows' words)
     int ntypes;                // type ids of the candidates are below this
     int grid;                  // workgroups (persistent)
 };
 size_t query_lds_bytes(int T, int c16, int mode, int maxC, int maxE, int maxTrg, int maxKmax,
                        int maxRows, int maxHK, int maxP, int ntypes);
+// LDS words of the stencil rows, which the k-th neighbour extraction reuses
+int query_row_words(int maxRows, int mode);
 hipError_t query_max_blocks_per_cu(int T, int c16, int mode, size_t lds, int *nb);
 hipError_t launch_query(const QueryLaunch &q, hipStream_t s);
 
