@@ -1246,9 +1246,9 @@ pp_status plan_symmetric(pp_ctx *c, Slot &sl, pp_cloud *cl, JobRun &r)
         return PP_OK;
     uint32_t minor = 0;
     {
-        // (resident workgroups as the register counts allow: 7 in the
+        // (resident workgroups as the register counts allow: 8 in the
         // pair-count mode, 6 in the hybrid mode)
-        const size_t gran = 512, lds_cu = 160 * 1024, cap = p.mode == 2 ? 6 : 7;
+        const size_t gran = 512, lds_cu = 160 * 1024, cap = p.mode == 2 ? 6 : 8;
         auto wgs = [&](int nrows, int nminor) {
             const size_t l = query_lds_bytes(r.T_req, 1, p.mode, std::max(p.C, 1),
                                              std::max(p.E, 1), std::max(p.ntrg, 1),

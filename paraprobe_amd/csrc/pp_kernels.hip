@@ -619,7 +619,8 @@ struct QArgs {
     int taskw, entw;  // QueryLaunch
 };
 
-__device__ inline int find_job(const uint32_t *__restrict__ off, int njobs, uint32_t g)
+template <typename Off>
+__device__ inline int find_job(const Off *__restrict__ off, int njobs, uint32_t g)
 {
     int lo = 0, hi = njobs;  // off[lo] <= g < off[hi]
     while (hi - lo > 1) {
@@ -648,6 +649,15 @@ __device__ inline uint32_t xcc_id()
 {
     return __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 0xFu;
 }
+
+// constant address space: a uniform read goes through the scalar cache, into
+// scalar registers (through a generic or global pointer it is a vector load of
+// every wave and a read of the first lane)
+typedef __attribute__((address_space(4))) JobDev CJobDev;
+typedef __attribute__((address_space(4))) Tile CTile;
+typedef const Tile *TilePtr;
+typedef __attribute__((address_space(4))) TilePtr CTilePtr;
+typedef __attribute__((address_space(4))) uint32_t cu32;
 
 typedef float fvec4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) const fvec4 gfvec4;
@@ -752,12 +762,12 @@ __device__ inline int category_of(float d2, float isc, float ioff1, float ioffa,
 // MODE 2: pair counts as in MODE 0 plus per-center histograms over the kNN
 // range only (see JobDev::HK); centers whose kNN range holds too few
 // neighbours are flagged for a MODE 1 rerun.
-// Resident waves per SIMD asked of the compiler for 8-center tiles: 7 in the
-// pair-count mode (71 VGPRs, no spills), 6 in the hybrid mode (77; 7 fits in 72
-// VGPRs with spills in the per-tile code: 0.3 % faster on the 20M-ion job,
-// 13 % slower on the 100M-ion one, whose tiles are cheaper).
+// Resident waves per SIMD asked of the compiler for 8-center tiles: 8 in the
+// pair-count mode (64 VGPRs; 4M ions, R 3 nm: 6.75 ms, with 7 waves 7.07), 6 in
+// the hybrid mode (7 fits, no faster on 20M ions and 1 % slower on
+// 100M, whose LDS holds 6 workgroups a CU).
 template <int T, bool C16, int MODE>
-__global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE == 2) ? 6 : 1) void k_query(QArgs a)
+__global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE == 2) ? 6 : 1) void k_query(QArgs a)
 {
     constexpr bool PC = MODE == 1;
     constexpr bool HY = MODE == 2;
@@ -783,6 +793,9 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
     // center's histogram (else -1)
     uint32_t *s_task = lds + L.total;
 
+    // job records, tile offsets and tiles, written before the launch: read
+    // through the scalar cache
+    const CJobDev *jobs = (const CJobDev *)(uintptr_t)a.jobs;
     int tid = threadIdx.x;
     int cur = -1;
     // tile queues (one counter per XCD); thread 0 keeps the grab state
@@ -805,16 +818,17 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
         __syncthreads();
         const uint32_t g = rfl(s_g);
         const bool done = g >= a.end_tile;
-        const int job = done ? -1 : (int)rfl((uint32_t)find_job(a.tile_off, a.njobs, g));
+        const int job = done ? -1 : find_job((const cu32 *)(uintptr_t)a.tile_off, a.njobs, g);
         // the tile: cell key, first center, center count, target-type slot
         uint32_t t_key = 0, t_first = 0, t_count = 0;
         int ts = 0;
         if (!done) {
-            const Tile *tp = a.tiles[job] + (g - a.tile_off[job]);
-            t_key = rfl(tp->key);
-            t_first = rfl(tp->first);
-            t_count = rfl((uint32_t)tp->count);
-            ts = (int)rfl(tp->pad);
+            const CTile *tp = (const CTile *)(uintptr_t)((const CTilePtr *)(uintptr_t)a.tiles)[job] +
+                              (g - ((const cu32 *)(uintptr_t)a.tile_off)[job]);
+            t_key = tp->key;
+            t_first = tp->first;
+            t_count = tp->count;
+            ts = (int)tp->pad;
         }
         // s_P holds the pair counts of one (job, center type)
         const int pkey = done ? -1 : job * kMaxTrg + ts;
@@ -822,7 +836,7 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
         if (pkey != cur || (!done && pending > 0x7FFFFFFFull)) {
             if (cur >= 0) {
                 // flush the accumulated pair counts and statistics
-                const JobDev &P0 = a.jobs[cur / kMaxTrg];
+                const CJobDev &P0 = jobs[cur / kMaxTrg];
                 const int n = P0.E * P0.C;
                 if (P0.families & (FAM_RDF | FAM_RIPK)) {
                     unsigned long long *dst = P0.P + (size_t)(cur % kMaxTrg) * n;
@@ -857,7 +871,7 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
             }
             if (done)
                 break;
-            const JobDev &J = a.jobs[job];
+            const CJobDev &J = jobs[job];
             if (cur < 0 || job != cur / kMaxTrg) {
                 if (!HY)
                     for (int i = tid; i < J.C; i += kBlock)
@@ -901,7 +915,7 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
         if (done)
             break;
 
-        const JobDev &J = a.jobs[job];
+        const CJobDev &J = jobs[job];
         const int cnt = (int)t_count;
         const uint32_t key = t_key;
         const int C = J.C, E = J.E, EC = E * C;
@@ -1105,9 +1119,13 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 7 : (T == 8 && MODE
                 cyr[c] = p.y;
                 czr[c] = p.z;
             }
-            const float R2 = J.R2;
-            const float isc = J.idx_scale, ioff = J.idx_off;
-            const float ioff1 = J.idx_off1, ioffa = J.idx_off1a, amb2 = J.amb2;
+            float R2 = J.R2;
+            float isc = J.idx_scale, ioffa = J.idx_off1a, amb2 = J.amb2;
+            const float ioff = J.idx_off, ioff1 = J.idx_off1;
+            // (a vector instruction with a scalar operand takes half as long
+            // again as one without: the loop's constants in vector registers,
+            // 20M ions 148.4 and 146.0 ms)
+            asm volatile("" : "+v"(R2), "+v"(isc), "+v"(ioffa), "+v"(amb2));
             const float Cm1f = (float)(C - 1);
             const bool rdf = (J.families & (FAM_RDF | FAM_RIPK)) != 0;
             const bool count_in = J.count_in != 0;
