@@ -826,7 +826,7 @@ void layout_tables(JobRun &r)
     r.o_kinfo = (o + 1) & ~(size_t)1;
     o = r.o_kinfo + 512;
     r.o_xrow = o;
-    o += 256;
+    o += r.sym_minor ? 256 + kMaxTrg : 0;
     r.o_ckoff = o;
     o += kMaxEnv;
     r.o_taskck = o;
@@ -936,13 +936,15 @@ void stage_tables(const JobRun &r, uint32_t *h)
     std::memcpy(&h[r.o_ttasks], p.trg_tasks.data(), p.trg_tasks.size() * 4);
     if (!p.kinfo.empty())
         std::memcpy(&h[r.o_kinfo], p.kinfo.data(), 512 * 4);
-    {
+    if (r.sym_minor) {
         int32_t *x = (int32_t *)&h[r.o_xrow];
         std::fill(x, x + 256, -1);
         int k = p.E;
         for (int s = 0; s < p.ntrg; ++s)
-            if ((r.sym_minor >> s) & 1u)
+            if ((r.sym_minor >> s) & 1u) {
                 x[p.trg_type[s]] = p.C * k++;
+                x[256 + s] = p.envoff[p.trg_type[s]];
+            }
     }
     if (!p.ckoff.empty())
         std::memcpy(&h[r.o_ckoff], p.ckoff.data(), kMaxEnv * 4);
@@ -1164,7 +1166,7 @@ int query_rows(const JobRun &r, int mode)
 // center types against sym_type.
 int pair_words(const JobRun &r, int mode)
 {
-    const int x = mode == 0 ? __builtin_popcount(r.sym_minor) : 0;
+    const int x = mode != 1 ? __builtin_popcount(r.sym_minor) : 0;
     return std::max((std::max(r.plan.E, 1) + x) * std::max(r.plan.C, 1), 1);
 }
 
@@ -1180,16 +1182,16 @@ int pair_words(const JobRun &r, int mode)
 // the own cell, the cells before it and the cells after it, and the other
 // candidates from a list without t along every row.  Kept off when the
 // longer row table would cost the kernel resident workgroups.
-// In the pair-count mode the pairs of t's centers with the centers of the other
-// types e that are both center and neighbour types go the same way: t's tiles,
-// which read e's ions over the full range anyway, add such a pair to e's row
-// as well (sym_minor), and e's few-center tiles read t's ions only where
-// non-centers ask for them (4M ions, 9 type pairs, R 3 nm: 20 % fewer
-// evaluations, 7.20 instead of 7.84 ms of query kernel).  The hybrid mode
-// keeps e's own full tiles: there the second add's test in every pair of the
-// loop, which runs at its register limit, cost more than the tiles saved (20M
-// ions, R 5 nm: 159 against 152 ms).  Left out when the rows would cost
-// resident workgroups, or when the in-ball total is counted pair by pair.
+// The pairs of t's centers with the centers of the other types e that are both
+// center and neighbour types go the same way: t's tiles, which read e's ions
+// over the full range anyway, count such a pair in a row of its own that is
+// added to both types' counts (sym_minor), and e's few-center tiles read t's
+// ions only where non-centers or their kNN range ask for them (20 %
+// fewer evaluations; whole calls: 4M ions, 9 type pairs, R 3 nm, pair counts 8.2
+// and 7.6 ms, with a row for both 6.78 and 6.63; 20M ions, R 5 nm, k to 100:
+// 151.1 and 148.3 ms).  Left out when the rows would cost resident workgroups
+// (100M ions, C 602: 349 ms of query kernel with five workgroups, 334 without
+// the rows and six), or when the in-ball total is counted pair by pair.
 pp_status plan_symmetric(pp_ctx *c, Slot &sl, pp_cloud *cl, JobRun &r)
 {
     r.sym_slot = -1;
@@ -1259,7 +1261,7 @@ pp_status plan_symmetric(pp_ctx *c, Slot &sl, pp_cloud *cl, JobRun &r)
         const size_t base = wgs((int)r.rows.size(), 0);
         if (wgs((int)nsr, 0) < base)
             return PP_OK;
-        for (int s = 0; s < p.ntrg && others && p.mode == 0 && !r.count_in; ++s)
+        for (int s = 0; s < p.ntrg && others && !r.count_in; ++s)
             if (s != bslot && p.envoff[p.trg_type[s]] >= 0 &&
                 cl->type_count[p.trg_type[s]] > 0)
                 minor |= 1u << s;

@@ -185,10 +185,11 @@ struct JobDev {
     // The other center types whose pairs with sym_type are counted from its
     // tiles (bit set over target slots; their ions lie in list O, s2_o being
     // its ion2surf): a pair of a center of sym_type and a center of such a
-    // type has one squared distance, so the tile of the former adds it to
-    // both types' pair-count rows (xrow[type]: the words from the tile's own
-    // rows to the row (type, sym_type), or -1).  Tiles of these types read
-    // list S only for its non-centers and their kNN range, then list O.
+    // type has one squared distance, so the tile of the former counts it once,
+    // in a row that is added to both types' pair counts (xrow[type]: the words
+    // from the tile's own rows to that row, or -1; xrow[256 + slot]: the
+    // type's own row among the tile's).  Tiles of these types read list S only
+    // for its non-centers and their kNN range, then list O.
     uint32_t sym_minor;
     const float *s2_o;
     const int32_t *xrow;

@@ -560,7 +560,7 @@ __host__ __device__ inline Lay make_layout(int T, int c16, int mode, int maxC, i
     L.envoff = o;  // per type id below ntypes
     o += al4(ntypes);
     L.xrow = o;  // per type id: its row against sym_type among the pair counts, or -1
-    o += mode == 0 ? al4(ntypes) : 0;
+    o += mode != 1 ? al4(ntypes) : 0;
     L.kinfo = o;
     o += mode == 2 ? 2 * al4(ntypes) : 0;
     L.ckoff = o;
@@ -845,17 +845,20 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
                         if (v)
                             global_add(&dst[i], (unsigned long long)v);
                     }
-                    if (MODE == 0 && cur % kMaxTrg == P0.sym_slot) {
-                        // the rows (other center type, sym_type)
+                    if (!PC && cur % kMaxTrg == P0.sym_slot) {
+                        // the pairs with the other types' centers, for both
                         int k = n;
                         const int es = P0.envoff[P0.sym_type];
                         for (uint32_t w = P0.sym_minor; w; w &= w - 1u, k += P0.C) {
-                            unsigned long long *dx =
-                                P0.P + (size_t)__builtin_ctz(w) * n + (size_t)es;
+                            const int sl = __builtin_ctz(w);
+                            unsigned long long *dx = P0.P + (size_t)sl * n + (size_t)es;
+                            unsigned long long *dy = dst + P0.xrow[256 + sl];
                             for (int i = tid; i < P0.C; i += kBlock) {
                                 const uint32_t v = s_P[k + i];
-                                if (v)
+                                if (v) {
                                     global_add(&dx[i], (unsigned long long)v);
+                                    global_add(&dy[i], (unsigned long long)v);
+                                }
                             }
                         }
                     }
@@ -878,9 +881,9 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
                         s_edges[i] = J.edges[i];
                 for (int i = tid; i < a.ntypes; i += kBlock)
                     s_envoff[i] = J.envoff[i];
-                if (MODE == 0)
+                if (!PC)
                     for (int i = tid; i < a.ntypes; i += kBlock)
-                        s_xrow[i] = J.xrow[i];
+                        s_xrow[i] = J.sym_minor ? J.xrow[i] : -1;
                 if (HY) {
                     for (int i = tid; i < 2 * a.ntypes; i += kBlock)
                         ((int32_t *)s_kinfo)[i] = J.kinfo[i];
@@ -906,7 +909,7 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
                 }
             }
             const int n =
-                (J.E + (MODE == 0 && ts == J.sym_slot ? __builtin_popcount(J.sym_minor) : 0)) * J.C;
+                (J.E + (!PC && ts == J.sym_slot ? __builtin_popcount(J.sym_minor) : 0)) * J.C;
             for (int i = tid; i < n; i += kBlock)
                 s_P[i] = 0u;
             cur = pkey;
@@ -925,7 +928,7 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
         // s_ns) of list S, the others along srows[s_ns, nsrows) of list O, in
         // the tiles of sym_type and (minor) of the types whose pairs with its
         // centers its tiles count
-        const bool minor = MODE == 0 && ((J.sym_minor >> ts) & 1u) != 0u;
+        const bool minor = !PC && ((J.sym_minor >> ts) & 1u) != 0u;
         const bool sym = !PC && (ts == J.sym_slot || minor);
         const int nrt = sym ? J.nsrows : nrows;
         const Row *rtab = sym ? J.srows : J.rows;
@@ -1168,7 +1171,7 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
             auto sweep = [&](auto KIND, const gfvec4 *__restrict__ pos, int rlo, int rhi,
                              uint32_t clo, uint32_t chi) {
             constexpr bool SY = !PC && decltype(KIND)::value == 1;
-            constexpr bool XS = MODE == 0 && decltype(KIND)::value == 2;
+            constexpr bool XS = !PC && decltype(KIND)::value == 2;
             typedef __attribute__((address_space(1))) const float gfloat;
             const gfloat *s2o = XS ? rflp((const gfloat *)J.s2_o) : nullptr;
             const int nch = (int)((chi - clo + kWave - 1) / kWave);
@@ -1242,12 +1245,15 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
                 // it costs two vector instructions per chunk)
                 int cin = (int)rfl(count_in ? 1u : 0u);
                 asm volatile("" : "+s"(cin));
-                // this candidate's pair-count row (only dereferenced when envok)
-                uint32_t *acc_row = (PC ? s_H : s_P) + woff;
-                // and its own type's row against sym_type, when it is a center
-                const int xr = XS ? s_xrow[ptype] : 0;
-                const bool xadd = XS && xr >= 0 && s2 >= R2;
-                uint32_t *x_row = s_P + xr;
+                // this candidate's pair-count row (only dereferenced when
+                // envok); a center of another type has a row of its own, which
+                // counts for both types
+                int prow = woff;
+                if (XS) {
+                    const int xr = s_xrow[ptype];
+                    prow = xr >= 0 && s2 >= R2 ? xr : woff;
+                }
+                uint32_t *acc_row = (PC ? s_H : s_P) + prow;
                 if (PC) {
                     // 1) all T squared distances (the reference's FP32 expression)
                     float d2[T];
@@ -1339,9 +1345,6 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
                                 __hip_atomic_fetch_add(acc_row + cat, 1u,
                                                        __ATOMIC_RELAXED,
                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
-                                if (xadd)
-                                    __hip_atomic_fetch_add(x_row + cat, 1u, __ATOMIC_RELAXED,
-                                                           __HIP_MEMORY_SCOPE_WORKGROUP);
                             }
                         }
                     }
@@ -1453,8 +1456,8 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
                 const int ns = (int)rfl((uint32_t)J.s_ns);
                 sweep(CInt<1>(), rflp((const gfvec4 *)J.pos_s), 0, ns, 0u, bs);
                 if (ns < nrt) {
-                    if (MODE == 0 && !minor && J.sym_minor != 0u)
-                        sweep(CInt<MODE == 0 ? 2 : 0>(), rflp((const gfvec4 *)J.pos_o), ns, nrt, bs,
+                    if (__builtin_expect(!PC && !minor && J.sym_minor != 0u, 0))
+                        sweep(CInt<PC ? 0 : 2>(), rflp((const gfvec4 *)J.pos_o), ns, nrt, bs,
                               ctot);
                     else
                         sweep(CInt<0>(), rflp((const gfvec4 *)J.pos_o), ns, nrt, bs, ctot);

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as O
-from paraprobe_amd import FAM_RDF, FAM_RIPK, Job, synth
+from paraprobe_amd import FAM_MKNN, FAM_RDF, FAM_RIPK, Job, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +50,28 @@ def test_cross_type_pairs_count_once_for_both(ctx, n, frac, tasks, surface):
     assert np.array_equal(got.ripk, want["ripk"])
     assert got.pairs_inball == st["inball"]
     assert got.centers_considered == st["considered"]
+
+
+@pytest.mark.parametrize("surface", ["frustum", "scattered"])
+@pytest.mark.parametrize("n,frac,tasks", CASES)
+def test_cross_type_pairs_hybrid(ctx, n, frac, tasks, surface):
+    """The same with k-th neighbours: in the hybrid mode (which some of the cases
+    take) the other types' tiles read the dominant type's ions over its kNN
+    range only."""
+    print(f"test_cross_type kNN n={n} types={len(frac)} {surface}", flush=True)
+    tip = synth.tip(n, 9, "frustum", 9.0, 5.0, 28.0 * n / 30_000 + 8.0, frac)
+    s2 = tip.ion2surf_sqr.copy()
+    if surface == "scattered":
+        s2 = np.random.default_rng(n + 1).uniform(0, 6, size=n).astype(np.float32)
+    job = Job(tasks, 0.0, 0.01, 1.7, FAM_RDF | FAM_RIPK | FAM_MKNN, kvalues=[1, 2, 5])
+    cloud = ctx.upload(tip.xyz, tip.types, s2)
+    try:
+        got = ctx.run(cloud, job)
+    finally:
+        cloud.free()
+    print(got.kernel, flush=True)
+    want, st = O.spatstat(tip.xyz, tip.types, s2, tasks, job.rmin, job.rincr, job.rmax,
+                          job.families, kvalues=job.kvalues)
+    for name in want:
+        assert np.array_equal(getattr(got, name), want[name]), name
+    assert got.pairs_inball == st["inball"]
