@@ -1145,6 +1145,16 @@ void fill_jobdev(JobRun &r)
     d.xrow = (const int32_t *)(r.tables + r.o_xrow);
 }
 
+// Workgroups of the query kernel that fit a CU's LDS, `lds` bytes of dynamic
+// LDS each: 160 KiB, handed out in units of 1280 bytes.  (The occupancy query
+// of the runtime rounds to 512: 20M ions, R 5 nm, k to 100 ran five workgroups
+// where it says six.)
+size_t lds_workgroups(size_t lds)
+{
+    const size_t unit = 1280, fixed = 16;  // the kernel's static words
+    return (size_t(160) << 10) / ((lds + fixed + unit - 1) / unit * unit);
+}
+
 // One more than the largest type id among a cloud's ions (the query kernel's
 // per-type tables hold that many entries).
 int type_span(const pp_cloud *cl)
@@ -1168,6 +1178,26 @@ int pair_words(const JobRun &r, int mode)
 {
     const int x = mode != 1 ? __builtin_popcount(r.sym_minor) : 0;
     return std::max((std::max(r.plan.E, 1) + x) * std::max(r.plan.C, 1), 1);
+}
+
+// Workgroups on a CU (6 at most, as its registers allow) of a job in the hybrid
+// mode with cells of Rmax/r, 1/ay of that in y and z, its rows those of
+// symmetric pair counting; 0 in the other modes.
+size_t hybrid_workgroups(const pp_cloud *cl, const JobPlan &p, int T, int r, int ay)
+{
+    if (p.mode != 2 || !(p.families & (PP_FAM_RDF | PP_FAM_RIPK)))
+        return 0;
+    const double w = (double)p.R / r * (1.0 + std::ldexp(1.0, -10));
+    const int nrows = 2 * (int)make_rows(w, w / ay, p.R).size() + 2;
+    int minor = -1;  // the other types that are center and neighbour types
+    for (int s = 0; s < p.ntrg; ++s)
+        minor += p.envoff[p.trg_type[s]] >= 0 && cl->type_count[p.trg_type[s]] > 0;
+    return std::min<size_t>(
+        6, lds_workgroups(query_lds_bytes(T, 1, 2, std::max(p.C, 1), std::max(p.E, 1),
+                                          std::max(p.ntrg, 1), p.kidx_len(), nrows,
+                                          std::max(p.HK, 1),
+                                          (p.E + std::max(minor, 0)) * std::max(p.C, 1),
+                                          type_span(cl))));
 }
 
 // Symmetric pair counting for a job with pair counts (RDF, RIPK) in the
@@ -1250,13 +1280,12 @@ pp_status plan_symmetric(pp_ctx *c, Slot &sl, pp_cloud *cl, JobRun &r)
     {
         // (resident workgroups as the register counts allow: 8 in the
         // pair-count mode, 6 in the hybrid mode)
-        const size_t gran = 512, lds_cu = 160 * 1024, cap = p.mode == 2 ? 6 : 8;
+        const size_t cap = p.mode == 2 ? 6 : 8;
         auto wgs = [&](int nrows, int nminor) {
-            const size_t l = query_lds_bytes(r.T_req, 1, p.mode, std::max(p.C, 1),
-                                             std::max(p.E, 1), std::max(p.ntrg, 1),
-                                             p.kidx_len(), nrows, std::max(p.HK, 1),
-                                             (p.E + nminor) * p.C, type_span(cl));
-            return std::min<size_t>(cap, lds_cu / ((l + gran - 1) / gran * gran));
+            return std::min(cap, lds_workgroups(query_lds_bytes(
+                                     r.T_req, 1, p.mode, std::max(p.C, 1), std::max(p.E, 1),
+                                     std::max(p.ntrg, 1), p.kidx_len(), nrows,
+                                     std::max(p.HK, 1), (p.E + nminor) * p.C, type_span(cl))));
         };
         const size_t base = wgs((int)r.rows.size(), 0);
         if (wgs((int)nsr, 0) < base)
@@ -1761,16 +1790,15 @@ pp_status launch_group(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std
             maxL = std::max(maxL, p->lmax);
             keff = std::max(keff, p->kmax);
         }
-        auto wgs = [&](size_t l) { return (size_t(160) << 10) / ((l + 511) / 512 * 512); };
         auto room = [&](size_t words) {
             const size_t l = lds + 4 * words;
-            return l <= c->lds_per_block && wgs(l) == wgs(lds);
+            return l <= c->lds_per_block && lds_workgroups(l) == lds_workgroups(lds);
         };
         for (int n : {std::min(maxL, 64), std::min(maxL, 8)})
             if (!taskw && room(4 * (size_t)n))
                 taskw = 4 * n;
-        const int need = ((c16 ? 2 : 1) * std::max(keff, 1) + 1) / 2;
-        if (need > query_row_words(maxRows, mode) / kWaves &&
+        const int need = ((c16 ? 2 : 1) * std::max(keff, 1) + 3) / 4;
+        if (maxC <= kEntryCats && need > query_row_words(maxRows, mode) / kWaves &&
             room((size_t)taskw + (size_t)kWaves * (size_t)need))
             entw = need;
     }
@@ -2022,15 +2050,24 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
         }
         runs[i].T_req = jT;
         p.ay = jAY > 0 ? jAY : tuneAY > 0 ? tuneAY : 1;
+        plan_hybrid(clouds[i], p, knn_factor);
         // the rule's cells of Rmax/4 and Rmax/2 are taken twice as long
         // along x in the lists jobs build for themselves (Rmax/2 by Rmax/4,
-        // Rmax by Rmax/2): the same stencil rows, each of half as many cells
+        // Rmax by Rmax/2): the same stencil rows, each of half as many cells.
+        // Cubes of Rmax/3 instead of Rmax/2 by Rmax/4, whose evaluations cost
+        // 2 % more, where their shorter row table leaves more workgroups on a
+        // CU (20M ions, R 5 nm: k to 10 120.5 and 123.2 ms of query kernel, k
+        // to 100, with five and six workgroups, 137.7 and 128.9)
         if (by_rule && tuneAY <= 0 && jAY <= 0 && (p.r == 4 || p.r == 2) &&
             !clouds[i]->resident) {
-            p.r /= 2;
-            p.ay = 2;
+            if (p.r == 4 && hybrid_workgroups(clouds[i], p, jT, 3, 1) >
+                                hybrid_workgroups(clouds[i], p, jT, 2, 2)) {
+                p.r = 3;
+            } else {
+                p.r /= 2;
+                p.ay = 2;
+            }
         }
-        plan_hybrid(clouds[i], p, knn_factor);
     }
     PP_HIP(c, hipSetDevice(c->device));
     // a non-resident cloud's cached cell list is rebuilt per width: hold it

@@ -572,8 +572,8 @@ __host__ __device__ inline Lay make_layout(int T, int c16, int mode, int maxC, i
     L.rowpre = o;  // per row its first index in the rows' concatenation
     o += al4(maxRows + 1);
     // after the main loop these words hold the entries of the k-th category
-    // extraction or, for k beyond what they hold, at their end per wavefront
-    // its k window (both uint16)
+    // extraction (bytes) or, for k beyond what they hold, at their end per
+    // wavefront its k window (uint16)
     if (mode && o < L.rows + kWinWords + 24)
         o = L.rows + kWinWords + 24;
     L.win = mode ? o - kWinWords : o;
@@ -1563,19 +1563,17 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
             // each mark to the k after it, and the group's 4 words, read
             // again, give the category.  The kernel's
             // times with one center, 2 categories a lane and a mark per
-            // category, as below, and now: 100 million ions, k to 20, 394 and
+            // category, as below, and so: 100 million ions, k to 20, 394 and
             // 334 ms (293 ms without any extraction); 20 million, k to 100,
-            // 153 and 147 ms (136).
+            // 153 and 147 ms (136); before later changes of the kernel.
             constexpr int UC = C16 ? 2 : 1;
             const int keff = want_k ? kmax : 1;  // entries per task and center
             const int ne = UC * keff;
-            // a wave's entries: in words of their own, or in the stencil
+            // a wave's entries, in words of their own, or in the stencil
             // rows' (free until the next tile) as far as these hold them
-            const int ewords =
-                a.entw > 0 ? a.entw : (L.cen - L.rows) / kWaves;
-            uint16_t *ent =
-                (uint16_t *)(a.entw > 0 ? s_task + a.taskw : s_rows) + 2 * ewords * wid;
-            const bool fits = ne <= 2 * ewords;
+            const int ewords = a.entw > 0 ? a.entw : (L.cen - L.rows) / kWaves;
+            uint8_t *ent = (uint8_t *)((a.entw > 0 ? s_task + a.taskw : s_rows) + ewords * wid);
+            const bool fits = ne <= 4 * ewords && C <= kEntryCats;
             const int nunit =
                 (want_k || want_1) && kb && fits ? (cnt + UC - 1) / UC : 0;
             for (int u = wid; u < nunit; u += kWaves) {
@@ -1636,7 +1634,7 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
                             const uint32_t sv = C16 ? (h ? sum >> 16 : sum & 0xFFFFu) : sum;
                             const uint32_t ev = C16 ? (h ? excl >> 16 : excl & 0xFFFFu) : excl;
                             if (sv != 0u && ev < (uint32_t)keff)
-                                ent[h * keff + (int)ev] = (uint16_t)((ca >> 2) + 1);
+                                ent[h * keff + (int)ev] = (uint8_t)((ca >> 2) + 1);
                         }
                         carry += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
                         tot0 = C16 ? carry & 0xFFFFu : carry;
@@ -1697,7 +1695,7 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
                     if (HY && ((shortm >> h) & 1u))
                         empty_rows(u * UC + h);
             }
-            // k beyond what the entries hold
+            // k beyond what the entries hold, and categories beyond their bytes
             for (int c = wid; c < cnt && !fits; c += kWaves) {
                 const int hoff = (C16 ? (c >> 1) : c) * (PC ? EC : HK);
                 const int sh = (C16 && (c & 1)) ? 16 : 0;

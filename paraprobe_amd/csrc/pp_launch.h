@@ -142,6 +142,9 @@ size_t query_lds_bytes(int T, int c16, int mode, int maxC, int maxE, int maxTrg,
                        int maxRows, int maxHK, int maxP, int ntypes);
 // LDS words of the stencil rows, which the k-th neighbour extraction reuses
 int query_row_words(int maxRows, int mode);
+// most categories of a job whose extraction uses them: an entry, the number of
+// a group of 4 categories, is a byte
+constexpr int kEntryCats = 4 * 254;
 hipError_t query_max_blocks_per_cu(int T, int c16, int mode, size_t lds, int *nb);
 hipError_t launch_query(const QueryLaunch &q, hipStream_t s);
 

@@ -9,6 +9,7 @@ from paraprobe_amd import FAM_1NN, FAM_CNTNB, FAM_MKNN, FAM_RDF, FAM_RIPK, Job, 
 
 pytestmark = pytest.mark.gpu
 
+ALL_PAIRS = synth.ALL_PAIRS
 ONE = [((1,), (2,))]
 MIX = [((1,), (1,)), ((1, 2), (1, 3)), ((3,), (2,)), ((1,), (1, 2, 3)), ((2,), (3,))]
 # (tasks, increment, ks): full-range and hybrid histograms follow from the k
@@ -18,10 +19,12 @@ CASES = [
     (ONE, 0.0023, list(range(1, 32))),
     (MIX, 0.01, list(range(1, 33))),
     (MIX, 0.004, [1, 2, 17, 33]),
-    (synth.ALL_PAIRS, 0.005, list(range(1, 21))),
-    (synth.ALL_PAIRS, 0.0051, [64, 65, 100]),
+    (ALL_PAIRS, 0.005, list(range(1, 21))),
+    (ALL_PAIRS, 0.0051, [64, 65, 100]),
     (MIX, 0.01, [1, 50, 300]),
     (ONE, 0.01, [2, 129, 700]),
+    # 1,268 categories: more than an entry's byte numbers
+    (ALL_PAIRS, 0.0015, [1, 20, 40]),
 ]
 
 
