@@ -1615,6 +1615,9 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
                     };
                     for (int i = lane; i < ne; i += kWave)
                         ent[i] = 0u;
+                    // (the fences keep the compiler from carrying a lane's own
+                    // stores over the other lanes' to its loads)
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                     uint32_t carry = 0u, tot0 = 0u, tot1 = need;
                     for (int cb = 0; cb < ck; cb += 4 * kWave) {
                         const int ca = cb + 4 * lane;
@@ -1649,6 +1652,7 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
                     // empty)
                     if (HY && (ckw >> 31))
                         shortm |= (tot0 < need ? 1u : 0u) | (tot1 < need ? 2u : 0u);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                     uint32_t last = 0u;
                     for (int i0 = 0; i0 < ne; i0 += kWave) {
                         const int i = i0 + lane;
