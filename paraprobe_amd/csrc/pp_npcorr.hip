@@ -78,6 +78,18 @@ __device__ inline uint32_t wave_scan(uint32_t v)
     return v;
 }
 
+// Inclusive running maximum over the 64 lanes, with the same moves.
+__device__ inline uint32_t wave_max(uint32_t v)
+{
+    v = __builtin_elementwise_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false));
+    v = __builtin_elementwise_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false));
+    v = __builtin_elementwise_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false));
+    v = __builtin_elementwise_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false));
+    v = __builtin_elementwise_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false));
+    v = __builtin_elementwise_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false));
+    return v;
+}
+
 // a value of one lane, the lane index being the same in the whole wave
 __device__ inline uint32_t lane_value(uint32_t v, int l)
 {
@@ -136,9 +148,11 @@ __global__ __launch_bounds__(256) void k_npcorr(NpcArgs a)
 {
     __shared__ uint4 s_buf[kWaves][kNpcCap];
     __shared__ uint32_t s_hist[kWaves][kNpcBuckets + 1];
+    __shared__ uint8_t s_mark[kWaves][kWave];
     const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
     uint4 *buf = s_buf[wid];
     uint32_t *hist = s_hist[wid];
+    uint8_t *mark = s_mark[wid];
     const uint64_t ci = (uint64_t)blockIdx.x * kWaves + wid;
     if (ci >= a.n)
         return;
@@ -147,39 +161,47 @@ __global__ __launch_bounds__(256) void k_npcorr(NpcArgs a)
     // considered: ion2surf >= fl32(R * R) (S.cpp:3846-3860)
     if (!(a.s2[ci] >= a.R2))
         return;
+    const int cx = cell_of(me.x, a.g.lo[0], a.g.inv_w, a.g.nx);
     const int cy = cell_of(me.y, a.g.lo[1], a.g.inv_w, a.g.ny);
     const int cz = cell_of(me.z, a.g.lo[2], a.g.inv_w, a.g.nz);
     // The candidates of a spherical shell ri <= d <= ro around the center in
     // a list with cell offsets cs: lane r < 25 takes the stencil row (dy, dz)
     // = (r % 5 - 2, r / 5 - 2) and keeps the x-cells where the shell can meet
     // the row -- one run, or two when the inner sphere cuts the row -- as
-    // candidate index ranges.  The bounds are exact in double on the cell
-    // boundaries lo + c * w (the same expression that bins the ions) and
-    // widened by 1e-4 w, far more than the rounding of the FP32 distance
-    // tests that decide membership.
-    const double px = me.x, py = me.y, pz = me.z, cw = a.g.w, margin = 1e-4 * cw;
-    auto rows_for = [&](const gcu32 *cs, double ri, double ro) {
+    // candidate index ranges.  In cells from the center's own cell, where
+    // single precision is off by some 1e-6 of a cell; the shell is widened by
+    // 1e-4 of one, far more than that and than the rounding of the FP32
+    // distance tests that decide membership.
+    // (In FP64 on absolute coordinates, and with a bisection over the ranges
+    // by lane shuffles below, 4M ions with K 99 took 20.1 ms, so 19.0.)
+    const float fx = (float)(((double)me.x - a.g.lo[0]) * a.g.inv_w - cx);
+    const float fy = (float)(((double)me.y - a.g.lo[1]) * a.g.inv_w - cy);
+    const float fz = (float)(((double)me.z - a.g.lo[2]) * a.g.inv_w - cz);
+    const float inv = (float)a.g.inv_w;
+    auto rows_for = [&](const gcu32 *cs, float ri, float ro) {
         Rows rw{0u, 0u, 0u, 0u};
-        const int y = cy + lane % 5 - 2, z = cz + lane / 5 - 2;
+        const int dy = lane % 5 - 2, dz = lane / 5 - 2;
+        const int y = cy + dy, z = cz + dz;
         if (lane >= 25 || y < 0 || y >= a.g.ny || z < 0 || z >= a.g.nz)
             return rw;
-        const double ylo = a.g.lo[1] + y * cw, zlo = a.g.lo[2] + z * cw;
-        const double hy0 = fmax(0.0, fmax(ylo - py, py - (ylo + cw)));
-        const double hz0 = fmax(0.0, fmax(zlo - pz, pz - (zlo + cw)));
-        const double hy1 = fmax(py - ylo, ylo + cw - py), hz1 = fmax(pz - zlo, zlo + cw - pz);
-        const double hmin2 = hy0 * hy0 + hz0 * hz0, hmax2 = hy1 * hy1 + hz1 * hz1;
-        ro += margin;
-        ri = ri > margin ? ri - margin : 0.0;
+        // the center's distance to the row's near and far faces
+        const float ya = fy - (float)dy, yb = (float)(dy + 1) - fy;
+        const float za = fz - (float)dz, zb = (float)(dz + 1) - fz;
+        const float hy0 = fmaxf(0.0f, fmaxf(-ya, -yb)), hz0 = fmaxf(0.0f, fmaxf(-za, -zb));
+        const float hy1 = fmaxf(ya, yb), hz1 = fmaxf(za, zb);
+        const float hmin2 = hy0 * hy0 + hz0 * hz0, hmax2 = hy1 * hy1 + hz1 * hz1;
+        ro = ro * inv + 1e-4f;
+        ri = fmaxf(ri * inv - 1e-4f, 0.0f);
         if (hmin2 > ro * ro)
             return rw;
-        const double xo = sqrt(ro * ro - hmin2);
-        const double xi2 = ri * ri - hmax2;
-        const double xi = xi2 > 0.0 ? sqrt(xi2) : 0.0;
-        auto cell = [&](double v) {
-            const double t = floor((v - a.g.lo[0]) * a.g.inv_w);
-            return t < 0.0 ? 0 : (t >= (double)a.g.nx ? a.g.nx - 1 : (int)t);
+        const float xo = __builtin_amdgcn_sqrtf(ro * ro - hmin2);
+        const float xi2 = ri * ri - hmax2;
+        const float xi = xi2 > 0.0f ? __builtin_amdgcn_sqrtf(xi2) : 0.0f;
+        auto cell = [&](float v) {
+            const int c = cx + (int)floorf(v);
+            return c < 0 ? 0 : (c >= a.g.nx ? a.g.nx - 1 : c);
         };
-        const int la = cell(px - xo), lb = cell(px - xi), ra = cell(px + xi), rb = cell(px + xo);
+        const int la = cell(fx - xo), lb = cell(fx - xi), ra = cell(fx + xi), rb = cell(fx + xo);
         const uint64_t row = ((uint64_t)z * a.g.ny + y) * a.g.nx;
         if (xi2 <= 0.0 || lb + 1 >= ra) {
             rw.b1 = cs[row + la];
@@ -242,26 +264,35 @@ __global__ __launch_bounds__(256) void k_npcorr(NpcArgs a)
                 f(q, ok);
             }
         } else {
-            auto at = [&](uint32_t sl) {
-                int k = 0;
-                for (int st = kWave / 2; st > 0; st >>= 1) {
-                    const uint32_t v = __shfl(excl, k + st, kWave);
-                    k = v <= sl ? k + st : k;
-                }
-                return __shfl(b, k, kWave) + (sl - __shfl(excl, k, kWave));
+            // the records of steps in order: every range marks its first
+            // candidate in the step, and a running maximum over the step
+            // gives each lane its range
+            const uint32_t base = b - excl;
+            uint32_t open = 0;  // the range, plus 1, that the step before ended in
+            auto at = [&](uint32_t w0) {
+                // (the fences keep the compiler from carrying a lane's own
+                // store over the other lanes' to its load)
+                mark[lane] = 0u;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                if (len > 0 && excl - w0 < (uint32_t)kWave)
+                    mark[excl - w0] = (uint8_t)(lane + 1);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                const uint32_t m =
+                    __builtin_elementwise_max(wave_max((uint32_t)mark[lane]), open);
+                open = lane_value(m, kWave - 1);
+                return __shfl(base, (int)m - 1, kWave) + w0 + (uint32_t)lane;
             };
             const uint32_t first = lane_value(b, (int)__builtin_ctzll(nonempty));
-            // (the searches run on every lane: a lane shuffle reads nothing
-            // from lanes that are switched off)
+            // (on every lane: a lane shuffle reads nothing from lanes that are
+            // switched off)
             bool cok = (uint32_t)lane < total;
-            const uint32_t j0 = at((uint32_t)lane);
+            const uint32_t j0 = at(0u);
             float4 cur = rec_at(p, cok ? j0 : first);
             for (uint32_t s0 = 0; s0 < total; s0 += kWave) {
                 const float4 q = cur;
                 const bool ok = cok;
-                const uint32_t sn = s0 + kWave + (uint32_t)lane;
-                cok = sn < total;
-                const uint32_t jn = at(sn);
+                cok = s0 + kWave + (uint32_t)lane < total;
+                const uint32_t jn = at(s0 + kWave);
                 cur = rec_at(p, cok ? jn : first);
                 f(q, ok);
             }
@@ -294,7 +325,7 @@ __global__ __launch_bounds__(256) void k_npcorr(NpcArgs a)
         const uint32_t bk = __float2uint_rz(d2 * inv_b2);
         return bk < bmax ? bk : bmax;
     };
-    const double reach = (double)a.maxlen * (1.0 + 0x1p-12);
+    const float reach = a.maxlen * (1.0f + 0x1p-12f);
     for (int t = 0; t < a.ntasks; ++t) {
         if (!((a.trg[t * 8 + (mt >> 5)] >> (mt & 31)) & 1u))
             continue;
@@ -326,7 +357,7 @@ __global__ __launch_bounds__(256) void k_npcorr(NpcArgs a)
             for (int q = lane; q <= kNpcBuckets; q += kWave)
                 hist[q] = 0;
             __builtin_amdgcn_wave_barrier();
-            const Rows ball = rows_for(ecs, 0.0, full ? reach : (double)r1 * (1.0 + 0x1p-12));
+            const Rows ball = rows_for(ecs, 0.0f, full ? reach : r1 * (1.0f + 0x1p-12f));
             sweep(ball, ep, [&](const float4 &q, bool ok) {
                 float u, v, w, d2;
                 if (ok && neighbour(q, u, v, w, d2))
@@ -378,11 +409,12 @@ __global__ __launch_bounds__(256) void k_npcorr(NpcArgs a)
         if (inb <= (uint32_t)kNpcCap) {
             // the selected bucket's candidates, ranked; they lie in the shell
             // of the bucket's distances
-            const double bw = 1.0 / (double)inv_b2;
-            const Rows shell = rows_for(ecs, sqrt(bsel * bw) * (1.0 - 0x1p-12),
-                                        (bsel == kNpcBuckets - 1 && full)
-                                            ? reach
-                                            : sqrt((bsel + 1) * bw) * (1.0 + 0x1p-12));
+            const float bw = __builtin_amdgcn_rcpf(inv_b2);
+            const Rows shell = rows_for(
+                ecs, __builtin_amdgcn_sqrtf((float)bsel * bw) * (1.0f - 0x1p-12f),
+                (bsel == kNpcBuckets - 1 && full)
+                    ? reach
+                    : __builtin_amdgcn_sqrtf((float)(bsel + 1) * bw) * (1.0f + 0x1p-12f));
             uint32_t cnt = 0;
             sweep(shell, ep, [&](const float4 &q, bool ok) {
                 float u = 0.f, v = 0.f, w = 0.f, d2 = 0.f;
@@ -418,7 +450,7 @@ __global__ __launch_bounds__(256) void k_npcorr(NpcArgs a)
             const uint32_t K = a.K;
             bool dropped = !self;
             uint32_t cnt = 0;
-            const Rows ball = rows_for(ecs, 0.0, reach);
+            const Rows ball = rows_for(ecs, 0.0f, reach);
             sweep(ball, ep, [&](const float4 &q, bool ok) {
                 float u = 0.f, v = 0.f, w = 0.f, d2 = 0.f;
                 bool take = ok && neighbour(q, u, v, w, d2);
