@@ -37,9 +37,9 @@ PLAIN_PEAK_OPS = 39.3e12    # without packed FP32: one wave-64 VALU instruction 
 FLOP_PER_EVAL = 8           # 3 sub + 3 mul + 2 add (no FMA: fp-contract off)
 OPS_PER_EVAL = 9            # the same plus the in-ball compare
 # HBM bytes of the query kernel per step of the 20M-ion headline job, from two
-# rocprofv3 --pmc runs of this script (FETCH_SIZE x 2 and WRITE_SIZE x 1, the
-# factors a 1 GiB device copy reads): 93.0 GB read + 10.5 GB written
-TRAFFIC_HEADLINE = 1.035e11
+# rocprofv3 --pmc runs of the job (FETCH_SIZE x 2 and WRITE_SIZE x 1, the
+# factors a 1 GiB device copy reads): 48.4 GB read + 9.3 GB written
+TRAFFIC_HEADLINE = 5.78e10
 TRAFFIC_SOURCE = "profiles/k_query_frustum20M_rdf_mknn100.md"
 # the same for the 100M-ion job's query launches: 161.3 GB read + 11.9 GB
 # written
