@@ -212,6 +212,8 @@ __global__ __launch_bounds__(256) void k_surftile(const float4 *__restrict__ ion
     // per triangle of the chunk, 24 floats: centre (3), half extent + delta
     // (3), box (6), vertex 1 (3), edges e0 and e1 (6), padding (3)
     __shared__ float4 s_r[256][6];
+    __shared__ float s_red[4][6];
+    __shared__ uint32_t s_cnt[4];
     const SurfTile tl = tiles[blockIdx.x];
     const int tid = threadIdx.x;
     const bool act = tid < (int)tl.count;
@@ -224,26 +226,72 @@ __global__ __launch_bounds__(256) void k_surftile(const float4 *__restrict__ ion
     const float qux = px + R, quy = py + R, quz = pz + R;
     constexpr float kGrow = 1.0f + 0x1p-18f;
     float best = RSQR, bestg = RSQR * kGrow;
+    // A chunk's triangles are first tested against the box of the tile's ions:
+    // one whose widened box lies farther from it than every lane's bound is
+    // not staged at all (the same bound as each lane's below, from a box that
+    // holds all of them, widened by delta / 4 for the rounding of its centre
+    // and half extents).  5M ions, 66,000 triangles: 2174 and with this 1600 us.
+    const int lane = tid & 63, wid = tid / 64;
+    float bc[3], bh[3];
+    {
+        float ext[6] = {px, py, pz, -px, -py, -pz};  // least coordinates, least negated ones
+        for (int k = 0; k < 6; ++k) {
+            float v = act ? ext[k] : __builtin_inff();
+            for (int d = 1; d < 64; d <<= 1)
+                v = fminf(v, __shfl_xor(v, d, 64));
+            if (lane == 0)
+                s_red[wid][k] = v;
+        }
+        __syncthreads();
+        for (int k = 0; k < 3; ++k) {
+            const float lo = fminf(fminf(s_red[0][k], s_red[1][k]),
+                                   fminf(s_red[2][k], s_red[3][k]));
+            const float hi = -fminf(fminf(s_red[0][3 + k], s_red[1][3 + k]),
+                                    fminf(s_red[2][3 + k], s_red[3][3 + k]));
+            bc[k] = 0.5f * (lo + hi);
+            bh[k] = 0.5f * (hi - lo) + 0.25f * delta;
+        }
+    }
+    float worst = RSQR * kGrow;  // the largest bound of the tile's lanes
     const uint32_t ts = __builtin_amdgcn_readfirstlane(tcellstart[tl.cell]);
     const uint32_t te = __builtin_amdgcn_readfirstlane(tcellstart[tl.cell + 1]);
     for (uint32_t base = ts; base < te; base += 256) {
-        const uint32_t m = __builtin_amdgcn_readfirstlane((te - base) < 256u ? (te - base) : 256u);
-        __syncthreads();
-        if ((uint32_t)tid < m) {
-            const uint64_t t = list[base + tid];
+        const uint32_t left = te - base;
+        float b0 = 0.f, b1 = 0.f, b2 = 0.f, b3 = 0.f, b4 = 0.f, b5 = 0.f;
+        bool keep = (uint32_t)tid < left;
+        uint64_t t = 0;
+        if (keep) {
+            t = list[base + tid];
             const float *bx = box + 6 * t;
-            const float b0 = bx[0], b1 = bx[1], b2 = bx[2], b3 = bx[3], b4 = bx[4], b5 = bx[5];
+            b0 = bx[0], b1 = bx[1], b2 = bx[2], b3 = bx[3], b4 = bx[4], b5 = bx[5];
+            const float gx =
+                fmaxf(fabsf(bc[0] - 0.5f * (b0 + b3)) - (0.5f * (b3 - b0) + delta) - bh[0], 0.f);
+            const float gy =
+                fmaxf(fabsf(bc[1] - 0.5f * (b1 + b4)) - (0.5f * (b4 - b1) + delta) - bh[1], 0.f);
+            const float gz =
+                fmaxf(fabsf(bc[2] - 0.5f * (b2 + b5)) - (0.5f * (b5 - b2) + delta) - bh[2], 0.f);
+            keep = !(gx * gx + gy * gy + gz * gz > worst);
+        }
+        const uint64_t km = __builtin_amdgcn_ballot_w64(keep);
+        if (lane == 0)
+            s_cnt[wid] = (uint32_t)__builtin_popcountll(km);
+        __syncthreads();  // (also: every lane is done with the chunk before)
+        const uint32_t c0 = s_cnt[0], c1 = s_cnt[1], c2 = s_cnt[2], c3 = s_cnt[3];
+        const uint32_t m = __builtin_amdgcn_readfirstlane(c0 + c1 + c2 + c3);
+        if (keep) {
+            const uint32_t at = (wid > 0 ? c0 : 0u) + (wid > 1 ? c1 : 0u) + (wid > 2 ? c2 : 0u) +
+                                (uint32_t)__builtin_popcountll(km & ((1ull << lane) - 1ull));
             const float *v = tri + 9 * t;
             const float v0 = v[0], v1 = v[1], v2 = v[2], v3 = v[3], v4 = v[4], v5 = v[5];
             const float v6 = v[6], v7 = v[7], v8 = v[8];
-            s_r[tid][0] = make_float4(0.5f * (b0 + b3), 0.5f * (b1 + b4), 0.5f * (b2 + b5),
-                                      0.5f * (b3 - b0) + delta);
-            s_r[tid][1] = make_float4(0.5f * (b4 - b1) + delta, 0.5f * (b5 - b2) + delta, b0, b1);
-            s_r[tid][2] = make_float4(b2, b3, b4, b5);
+            s_r[at][0] = make_float4(0.5f * (b0 + b3), 0.5f * (b1 + b4), 0.5f * (b2 + b5),
+                                     0.5f * (b3 - b0) + delta);
+            s_r[at][1] = make_float4(0.5f * (b4 - b1) + delta, 0.5f * (b5 - b2) + delta, b0, b1);
+            s_r[at][2] = make_float4(b2, b3, b4, b5);
             // vertex 1 and the two edges as the reference forms them
-            s_r[tid][3] = make_float4(v0, v1, v2, v3 - v0);
-            s_r[tid][4] = make_float4(v4 - v1, v5 - v2, v6 - v0, v7 - v1);
-            s_r[tid][5] = make_float4(v8 - v2, 0.f, 0.f, 0.f);
+            s_r[at][3] = make_float4(v0, v1, v2, v3 - v0);
+            s_r[at][4] = make_float4(v4 - v1, v5 - v2, v6 - v0, v7 - v1);
+            s_r[at][5] = make_float4(v8 - v2, 0.f, 0.f, 0.f);
         }
         __syncthreads();
         for (uint32_t j = 0; j < m; ++j) {
@@ -268,6 +316,15 @@ __global__ __launch_bounds__(256) void k_surftile(const float4 *__restrict__ ion
                     }
                 }
             }
+        }
+        if (base + 256 < te) {
+            float w = act ? bestg : 0.f;
+            for (int d = 1; d < 64; d <<= 1)
+                w = fmaxf(w, __shfl_xor(w, d, 64));
+            if (lane == 0)
+                s_red[wid][0] = w;
+            __syncthreads();
+            worst = fmaxf(fmaxf(s_red[0][0], s_red[1][0]), fmaxf(s_red[2][0], s_red[3][0]));
         }
     }
     if (act)
