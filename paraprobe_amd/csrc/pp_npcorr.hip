@@ -190,7 +190,7 @@ __global__ __launch_bounds__(256) void k_npcorr(NpcArgs a)
         const float hy0 = fmaxf(0.0f, fmaxf(-ya, -yb)), hz0 = fmaxf(0.0f, fmaxf(-za, -zb));
         const float hy1 = fmaxf(ya, yb), hz1 = fmaxf(za, zb);
         const float hmin2 = hy0 * hy0 + hz0 * hz0, hmax2 = hy1 * hy1 + hz1 * hz1;
-        ro = ro * inv + 1e-4f;
+        ro = fminf(ro * inv + 1e-4f, 1e9f);  // (a whole row, also where R * R overflows)
         ri = fmaxf(ri * inv - 1e-4f, 0.0f);
         if (hmin2 > ro * ro)
             return rw;
@@ -409,12 +409,14 @@ __global__ __launch_bounds__(256) void k_npcorr(NpcArgs a)
         if (inb <= (uint32_t)kNpcCap) {
             // the selected bucket's candidates, ranked; they lie in the shell
             // of the bucket's distances
-            const float bw = __builtin_amdgcn_rcpf(inv_b2);
-            const Rows shell = rows_for(
-                ecs, __builtin_amdgcn_sqrtf((float)bsel * bw) * (1.0f - 0x1p-12f),
-                (bsel == kNpcBuckets - 1 && full)
-                    ? reach
-                    : __builtin_amdgcn_sqrtf((float)(bsel + 1) * bw) * (1.0f + 0x1p-12f));
+            // (in FP64: v_rcp_f32 and v_sqrt_f32 take subnormal numbers for
+            // zero, which the width of a bucket is for Rmax near 1e-18)
+            const double bw = 1.0 / (double)inv_b2;
+            const Rows shell =
+                rows_for(ecs, (float)(sqrt(bsel * bw) * (1.0 - 0x1p-12)),
+                         (bsel == kNpcBuckets - 1 && full)
+                             ? reach
+                             : (float)(sqrt((bsel + 1) * bw) * (1.0 + 0x1p-12)));
             uint32_t cnt = 0;
             sweep(shell, ep, [&](const float4 &q, bool ok) {
                 float u = 0.f, v = 0.f, w = 0.f, d2 = 0.f;
