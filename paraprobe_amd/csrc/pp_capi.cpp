@@ -1180,6 +1180,12 @@ int pair_words(const JobRun &r, int mode)
     return std::max((std::max(r.plan.E, 1) + x) * std::max(r.plan.C, 1), 1);
 }
 
+// LDS words of the table of those other center types' rows, for type ids below
+// ntypes, where a job of the launch has any.
+int cross_words(bool any, int ntypes) { return any ? (ntypes + 3) & ~3 : 0; }
+
+bool has_cross(const JobRun &r, int mode) { return mode != 1 && r.sym_minor != 0; }
+
 // Workgroups on a CU (6 at most, as its registers allow) of a job in the hybrid
 // mode with cells of Rmax/r, 1/ay of that in y and z, its rows those of
 // symmetric pair counting; 0 in the other modes.
@@ -1196,7 +1202,8 @@ size_t hybrid_workgroups(const pp_cloud *cl, const JobPlan &p, int T, int r, int
         6, lds_workgroups(query_lds_bytes(T, 1, 2, std::max(p.C, 1), std::max(p.E, 1),
                                           std::max(p.ntrg, 1), p.kidx_len(), nrows,
                                           std::max(p.HK, 1),
-                                          (p.E + std::max(minor, 0)) * std::max(p.C, 1),
+                                          (p.E + std::max(minor, 0)) * std::max(p.C, 1) +
+                                              cross_words(minor > 0, type_span(cl)),
                                           type_span(cl))));
 }
 
@@ -1222,6 +1229,9 @@ size_t hybrid_workgroups(const pp_cloud *cl, const JobPlan &p, int T, int r, int
 // 151.1 and 148.3 ms).  Left out when the rows would cost resident workgroups
 // (100M ions, C 602: 349 ms of query kernel with five workgroups, 334 without
 // the rows and six), or when the in-ball total is counted pair by pair.
+// Neither of the two is taken where its layout with 32-bit counters, which
+// run_jobs asks of every job, would not fit the LDS: a job that runs without
+// them is not refused for them.
 pp_status plan_symmetric(pp_ctx *c, Slot &sl, pp_cloud *cl, JobRun &r)
 {
     r.sym_slot = -1;
@@ -1281,20 +1291,27 @@ pp_status plan_symmetric(pp_ctx *c, Slot &sl, pp_cloud *cl, JobRun &r)
         // (resident workgroups as the register counts allow: 8 in the
         // pair-count mode, 6 in the hybrid mode)
         const size_t cap = p.mode == 2 ? 6 : 8;
+        auto bytes = [&](int T, int c16, int nrows, int nminor) {
+            return query_lds_bytes(T, c16, p.mode, std::max(p.C, 1), std::max(p.E, 1),
+                                   std::max(p.ntrg, 1), p.kidx_len(), nrows, std::max(p.HK, 1),
+                                   (p.E + nminor) * p.C + cross_words(nminor > 0, type_span(cl)),
+                                   type_span(cl));
+        };
         auto wgs = [&](int nrows, int nminor) {
-            return std::min(cap, lds_workgroups(query_lds_bytes(
-                                     r.T_req, 1, p.mode, std::max(p.C, 1), std::max(p.E, 1),
-                                     std::max(p.ntrg, 1), p.kidx_len(), nrows,
-                                     std::max(p.HK, 1), (p.E + nminor) * p.C, type_span(cl))));
+            return std::min(cap, lds_workgroups(bytes(r.T_req, 1, nrows, nminor)));
+        };
+        auto fits = [&](int nrows, int nminor) {
+            return bytes(std::min(r.T_req, 8), 0, nrows, nminor) <= c->lds_per_block;
         };
         const size_t base = wgs((int)r.rows.size(), 0);
-        if (wgs((int)nsr, 0) < base)
+        if (wgs((int)nsr, 0) < base || !fits((int)nsr, 0))
             return PP_OK;
         for (int s = 0; s < p.ntrg && others && !r.count_in; ++s)
             if (s != bslot && p.envoff[p.trg_type[s]] >= 0 &&
                 cl->type_count[p.trg_type[s]] > 0)
                 minor |= 1u << s;
-        if (minor && wgs((int)nsr, __builtin_popcount(minor)) < base)
+        const int nminor = __builtin_popcount(minor);
+        if (minor && (wgs((int)nsr, nminor) < base || !fits((int)nsr, nminor)))
             minor = 0;
     }
     uint32_t smask[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -1654,6 +1671,7 @@ pp_status launch_group(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std
     if (nj == 0)
         return PP_OK;
     int maxC = 1, maxE = 1, maxTrg = 1, maxK = 0, maxRows = 1, maxHK = 1, maxP = 1, ntypes = 1;
+    bool cross = false;
     uint32_t maxcand = 0;
     for (int q = 0; q < nj; ++q) {
         const JobRun &r = runs[ids[q]];
@@ -1666,9 +1684,11 @@ pp_status launch_group(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std
         if (mode == 2)
             maxHK = std::max(maxHK, p.HK);
         maxP = std::max(maxP, pair_words(r, mode));
+        cross = cross || has_cross(r, mode);
         ntypes = std::max(ntypes, type_span(r.cloud));
         maxcand = std::max(maxcand, r.h_counts[2]);
     }
+    maxP += cross_words(cross, ntypes);
     const int c16 = maxcand < 65535u ? 1 : 0;
     const size_t lds =
         query_lds_bytes(T, c16, mode, maxC, maxE, maxTrg, maxK, maxRows, maxHK, maxP, ntypes);
@@ -2143,7 +2163,8 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
         auto need = [&](int t) {
             return query_lds_bytes(t, 0, p.mode, std::max(p.C, 1), std::max(p.E, 1),
                                    std::max(p.ntrg, 1), p.kidx_len(), query_rows(r, p.mode),
-                                   std::max(p.HK, 1), pair_words(r, p.mode),
+                                   std::max(p.HK, 1), pair_words(r, p.mode) +
+                                       cross_words(has_cross(r, p.mode), type_span(r.cloud)),
                                    type_span(r.cloud));
         };
         while (need(r.T_req) > c->lds_per_block && r.T_req > 8)
@@ -2244,6 +2265,7 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
     auto lds_of = [&](const std::vector<int> &ids, int mode, int T, int c16) {
         int maxC = 1, maxE = 1, maxTrg = 1, maxK = 0, maxRows = 1, maxHK = 1, maxP = 1,
             ntypes = 1;
+        bool cross = false;
         for (int i : ids) {
             const JobPlan &p = runs[i].plan;
             maxC = std::max(maxC, p.C);
@@ -2254,10 +2276,11 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
             if (mode == 2)
                 maxHK = std::max(maxHK, p.HK);
             maxP = std::max(maxP, pair_words(runs[i], mode));
+            cross = cross || has_cross(runs[i], mode);
             ntypes = std::max(ntypes, type_span(runs[i].cloud));
         }
-        return query_lds_bytes(T, c16, mode, maxC, maxE, maxTrg, maxK, maxRows, maxHK, maxP,
-                               ntypes);
+        return query_lds_bytes(T, c16, mode, maxC, maxE, maxTrg, maxK, maxRows, maxHK,
+                               maxP + cross_words(cross, ntypes), ntypes);
     };
     struct Group {
         int mode, T, c16;

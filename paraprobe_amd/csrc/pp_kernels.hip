@@ -559,8 +559,6 @@ __host__ __device__ inline Lay make_layout(int T, int c16, int mode, int maxC, i
     o += mode == 2 ? 0 : al4(maxC);
     L.envoff = o;  // per type id below ntypes
     o += al4(ntypes);
-    L.xrow = o;  // per type id: its row against sym_type among the pair counts, or -1
-    o += mode != 1 ? al4(ntypes) : 0;
     L.kinfo = o;
     o += mode == 2 ? 2 * al4(ntypes) : 0;
     L.ckoff = o;
@@ -583,6 +581,9 @@ __host__ __device__ inline Lay make_layout(int T, int c16, int mode, int maxC, i
     o += al4(T);
     L.P = o;
     o += al4(maxP);  // pair counts of one center type (tiles hold one type)
+    // at their end, where a job of the launch has cross-type rows: per type id
+    // its row against sym_type among the pair counts, or -1
+    L.xrow = o - al4(ntypes);
     L.H = o;
     const int hc = c16 ? (T + 1) / 2 : T;
     // (and 4 words behind them: the extraction reads 4 categories at a time)
@@ -884,9 +885,9 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
                         s_edges[i] = J.edges[i];
                 for (int i = tid; i < a.ntypes; i += kBlock)
                     s_envoff[i] = J.envoff[i];
-                if (!PC)
+                if (!PC && J.sym_minor)
                     for (int i = tid; i < a.ntypes; i += kBlock)
-                        s_xrow[i] = J.sym_minor ? J.xrow[i] : -1;
+                        s_xrow[i] = J.xrow[i];
                 if (HY) {
                     for (int i = tid; i < 2 * a.ntypes; i += kBlock)
                         ((int32_t *)s_kinfo)[i] = J.kinfo[i];

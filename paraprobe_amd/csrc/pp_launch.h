@@ -132,7 +132,9 @@ struct QueryLaunch {
     int mode;                  // 0 pair counts, 1 full-range per-center, 2 hybrid
     // maxKmax: the largest kmax of the jobs whose k are not 1..kmax (0: none)
     int maxC, maxE, maxTrg, maxKmax, maxRows, maxHK;
-    int maxP;                  // LDS words of a tile's pair-count rows (JobDev::xrow's included)
+    // LDS words of a tile's pair-count rows (JobDev::xrow's included) and, where
+    // a job has rows of that kind, of their table (ntypes, in whole 4 words)
+    int maxP;
     int taskw, entw;           // further LDS words: of the tasks' table (4 a task), and a wave's
                                // of the k-th neighbour entries (0: in the stencil rows' words)
     int ntypes;                // type ids of the candidates are below this
