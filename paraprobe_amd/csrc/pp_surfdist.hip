@@ -12,6 +12,8 @@
 // grid (each into every cell its R-inflated box touches) and one thread per
 // ion tests the triangles of its own cell with the reference's exact overlap
 // test and FP32 expression (no contraction, IEEE division).
+#include <algorithm>
+
 #include "pp_launch.h"
 
 #pragma clang fp contract(off)
@@ -144,33 +146,33 @@ __global__ __launch_bounds__(256) void k_tribox(const float *__restrict__ tri, u
                                                 float R, GridGeom g, float *__restrict__ box,
                                                 uint32_t *__restrict__ count)
 {
-    const uint64_t i = (uint64_t)blockIdx.x * 4u + threadIdx.x / 64u;
-    if (i >= ntri)
-        return;
-    const float *t = tri + 9 * i;
-    float b[6];
-    for (int k = 0; k < 3; ++k) {
-        b[k] = fminf(fminf(t[k], t[3 + k]), t[6 + k]);
-        b[3 + k] = fmaxf(fmaxf(t[k], t[3 + k]), t[6 + k]);
+    const uint64_t i0 = (uint64_t)blockIdx.x * 4u + threadIdx.x / 64u;
+    for (uint64_t i = i0; i < ntri; i += (uint64_t)gridDim.x * 4u) {
+        const float *t = tri + 9 * i;
+        float b[6];
+        for (int k = 0; k < 3; ++k) {
+            b[k] = fminf(fminf(t[k], t[3 + k]), t[6 + k]);
+            b[3 + k] = fmaxf(fmaxf(t[k], t[3 + k]), t[6 + k]);
+        }
+        if ((threadIdx.x & 63u) == 0u)
+            for (int k = 0; k < 6; ++k)
+                box[6 * i + k] = b[k];
+        int lo[3], hi[3];
+        tri_cells(b, R, g, lo, hi);
+        each_cell(g, lo, hi, [&](uint64_t c) { atomicAdd(&count[c], 1u); });
     }
-    if ((threadIdx.x & 63u) == 0u)
-        for (int k = 0; k < 6; ++k)
-            box[6 * i + k] = b[k];
-    int lo[3], hi[3];
-    tri_cells(b, R, g, lo, hi);
-    each_cell(g, lo, hi, [&](uint64_t c) { atomicAdd(&count[c], 1u); });
 }
 
 __global__ __launch_bounds__(256) void k_trifill(const float *__restrict__ box, uint64_t ntri,
                                                  float R, GridGeom g, uint32_t *__restrict__ cursor,
                                                  uint32_t *__restrict__ list)
 {
-    const uint64_t i = (uint64_t)blockIdx.x * 4u + threadIdx.x / 64u;
-    if (i >= ntri)
-        return;
-    int lo[3], hi[3];
-    tri_cells(box + 6 * i, R, g, lo, hi);
-    each_cell(g, lo, hi, [&](uint64_t c) { list[atomicAdd(&cursor[c], 1u)] = (uint32_t)i; });
+    const uint64_t i0 = (uint64_t)blockIdx.x * 4u + threadIdx.x / 64u;
+    for (uint64_t i = i0; i < ntri; i += (uint64_t)gridDim.x * 4u) {
+        int lo[3], hi[3];
+        tri_cells(box + 6 * i, R, g, lo, hi);
+        each_cell(g, lo, hi, [&](uint64_t c) { list[atomicAdd(&cursor[c], 1u)] = (uint32_t)i; });
+    }
 }
 
 // Ions into cell order: (x, y, z, original index as bits).
@@ -346,12 +348,19 @@ hipError_t launch_fill(float *out, uint64_t n, float v, hipStream_t s)
     return hipGetLastError();
 }
 
+// Workgroups for ntri triangles, a wavefront each: a grid holds at most 2^32
+// threads, so beyond 2^20 workgroups (4 million triangles) they take several.
+static unsigned tri_blocks(uint64_t ntri)
+{
+    return std::min(blocks_for(ntri, 4), 1u << 20);
+}
+
 hipError_t launch_tribox(const float *tri, uint64_t ntri, float R, GridGeom g, float *box,
                          uint32_t *count, hipStream_t s)
 {
     if (ntri == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(k_tribox, dim3(blocks_for(ntri, 4)), dim3(256), 0, s, tri, ntri, R, g,
+    hipLaunchKernelGGL(k_tribox, dim3(tri_blocks(ntri)), dim3(256), 0, s, tri, ntri, R, g,
                        box, count);
     return hipGetLastError();
 }
@@ -361,7 +370,7 @@ hipError_t launch_trifill(const float *box, uint64_t ntri, float R, GridGeom g, 
 {
     if (ntri == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(k_trifill, dim3(blocks_for(ntri, 4)), dim3(256), 0, s, box, ntri, R, g,
+    hipLaunchKernelGGL(k_trifill, dim3(tri_blocks(ntri)), dim3(256), 0, s, box, ntri, R, g,
                        cursor, list);
     return hipGetLastError();
 }
