@@ -121,20 +121,20 @@ __device__ inline void tri_cells(const float *box, float R, const GridGeom &g, i
     }
 }
 
-// The cells [lo, hi] of one triangle, a cell a lane: f(cell index).  One
-// wavefront per triangle: its lanes' counters are different ones, side by side
+// The cells [lo, hi] of one triangle, a cell a lane of its G: f(cell index).
+// A triangle's lanes' counters are different ones, side by side
 // along x.  (With a triangle per lane, neighbouring triangles of a mesh take
 // the same cells in the same step, and the counters' atomics wait for each
-// other: 66,000 triangles in 5 million ions, k_tribox 583 and now 183 us,
-// k_trifill 667 and 233 us.)
-template <typename F>
+// other: 66,000 triangles in 5 million ions, k_tribox 583 and with 64 lanes a
+// triangle 183 us, k_trifill 667 and 233 us.)
+template <int G, typename F>
 __device__ inline void each_cell(const GridGeom &g, const int lo[3], const int hi[3], F f)
 {
     if (hi[0] < lo[0] || hi[1] < lo[1] || hi[2] < lo[2])
         return;
     const uint32_t dx = (uint32_t)(hi[0] - lo[0] + 1), dy = (uint32_t)(hi[1] - lo[1] + 1);
     const uint32_t nc = dx * dy * (uint32_t)(hi[2] - lo[2] + 1);
-    for (uint32_t c = threadIdx.x & 63u; c < nc; c += 64u) {
+    for (uint32_t c = threadIdx.x & (G - 1u); c < nc; c += (uint32_t)G) {
         const uint32_t r = c / dx;
         const uint32_t x = (uint32_t)lo[0] + (c - r * dx), z = (uint32_t)lo[2] + r / dy;
         const uint32_t y = (uint32_t)lo[1] + r % dy;
@@ -142,36 +142,40 @@ __device__ inline void each_cell(const GridGeom &g, const int lo[3], const int h
     }
 }
 
+template <int G>
 __global__ __launch_bounds__(256) void k_tribox(const float *__restrict__ tri, uint64_t ntri,
                                                 float R, GridGeom g, float *__restrict__ box,
                                                 uint32_t *__restrict__ count)
 {
-    const uint64_t i0 = (uint64_t)blockIdx.x * 4u + threadIdx.x / 64u;
-    for (uint64_t i = i0; i < ntri; i += (uint64_t)gridDim.x * 4u) {
+    constexpr uint32_t kPer = 256u / G;  // triangles of a workgroup
+    const uint64_t i0 = (uint64_t)blockIdx.x * kPer + threadIdx.x / G;
+    for (uint64_t i = i0; i < ntri; i += (uint64_t)gridDim.x * kPer) {
         const float *t = tri + 9 * i;
         float b[6];
         for (int k = 0; k < 3; ++k) {
             b[k] = fminf(fminf(t[k], t[3 + k]), t[6 + k]);
             b[3 + k] = fmaxf(fmaxf(t[k], t[3 + k]), t[6 + k]);
         }
-        if ((threadIdx.x & 63u) == 0u)
+        if ((threadIdx.x & (G - 1u)) == 0u)
             for (int k = 0; k < 6; ++k)
                 box[6 * i + k] = b[k];
         int lo[3], hi[3];
         tri_cells(b, R, g, lo, hi);
-        each_cell(g, lo, hi, [&](uint64_t c) { atomicAdd(&count[c], 1u); });
+        each_cell<G>(g, lo, hi, [&](uint64_t c) { atomicAdd(&count[c], 1u); });
     }
 }
 
+template <int G>
 __global__ __launch_bounds__(256) void k_trifill(const float *__restrict__ box, uint64_t ntri,
                                                  float R, GridGeom g, uint32_t *__restrict__ cursor,
                                                  uint32_t *__restrict__ list)
 {
-    const uint64_t i0 = (uint64_t)blockIdx.x * 4u + threadIdx.x / 64u;
-    for (uint64_t i = i0; i < ntri; i += (uint64_t)gridDim.x * 4u) {
+    constexpr uint32_t kPer = 256u / G;  // triangles of a workgroup
+    const uint64_t i0 = (uint64_t)blockIdx.x * kPer + threadIdx.x / G;
+    for (uint64_t i = i0; i < ntri; i += (uint64_t)gridDim.x * kPer) {
         int lo[3], hi[3];
         tri_cells(box + 6 * i, R, g, lo, hi);
-        each_cell(g, lo, hi, [&](uint64_t c) { list[atomicAdd(&cursor[c], 1u)] = (uint32_t)i; });
+        each_cell<G>(g, lo, hi, [&](uint64_t c) { list[atomicAdd(&cursor[c], 1u)] = (uint32_t)i; });
     }
 }
 
@@ -348,11 +352,22 @@ hipError_t launch_fill(float *out, uint64_t n, float v, hipStream_t s)
     return hipGetLastError();
 }
 
-// Workgroups for ntri triangles, a wavefront each: a grid holds at most 2^32
-// threads, so beyond 2^20 workgroups (4 million triangles) they take several.
-static unsigned tri_blocks(uint64_t ntri)
+// Lanes that take a triangle's cells: 4 where R is less than half a cell, so
+// that a small triangle touches 8 cells at most and mostly one or two, else a
+// wavefront.  (Whole calls with 1, 4 and 64 lanes, 30,000 ions in cells of 2.5:
+// 200,000 triangles of 0.02, R 0.5: 1.80, 1.56 and 2.25 ms, R 1: 3.00, 2.21 and
+// 2.89, of 1, R 1: 6.87, 5.07 and 5.51; beyond the line, R 2: 11.7, 7.76 and 6.74;
+// 20,000 of 0.3, R 4: 3.22, 2.01 and 1.10.)
+static int tri_lanes(float R, const GridGeom &g)
 {
-    return std::min(blocks_for(ntri, 4), 1u << 20);
+    return 2.0 * (double)R * g.inv_w < 1.0 ? 4 : 64;
+}
+
+// Workgroups for ntri triangles of `lanes` lanes each: a grid holds at most
+// 2^32 threads, so beyond 2^20 workgroups a lane group takes several.
+static unsigned tri_blocks(uint64_t ntri, int lanes)
+{
+    return std::min(blocks_for(ntri, 256u / (unsigned)lanes), 1u << 20);
 }
 
 hipError_t launch_tribox(const float *tri, uint64_t ntri, float R, GridGeom g, float *box,
@@ -360,8 +375,9 @@ hipError_t launch_tribox(const float *tri, uint64_t ntri, float R, GridGeom g, f
 {
     if (ntri == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(k_tribox, dim3(tri_blocks(ntri)), dim3(256), 0, s, tri, ntri, R, g,
-                       box, count);
+    const int lanes = tri_lanes(R, g);
+    hipLaunchKernelGGL((lanes == 4 ? k_tribox<4> : k_tribox<64>), dim3(tri_blocks(ntri, lanes)),
+                       dim3(256), 0, s, tri, ntri, R, g, box, count);
     return hipGetLastError();
 }
 
@@ -370,8 +386,9 @@ hipError_t launch_trifill(const float *box, uint64_t ntri, float R, GridGeom g, 
 {
     if (ntri == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(k_trifill, dim3(tri_blocks(ntri)), dim3(256), 0, s, box, ntri, R, g,
-                       cursor, list);
+    const int lanes = tri_lanes(R, g);
+    hipLaunchKernelGGL((lanes == 4 ? k_trifill<4> : k_trifill<64>), dim3(tri_blocks(ntri, lanes)),
+                       dim3(256), 0, s, box, ntri, R, g, cursor, list);
     return hipGetLastError();
 }
 

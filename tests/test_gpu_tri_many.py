@@ -29,3 +29,19 @@ def test_many_triangles(ctx, log2):
     want = np.asarray(O.ion2surf(xyz, near.reshape(14, 9), R), np.float32)
     assert (want < R * R).any()
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("R", [0.3, 2.5, 2.54])
+@pytest.mark.parametrize("ntri", [1, 63, 64, 65, 4_099])
+def test_small_triangles(ctx, ntri, R):
+    """Cells of about 5.04: a group of lanes per triangle where R is less than
+    half of that, a wavefront from there on."""
+    print(f"test_small_triangles ntri={ntri} R={R}", flush=True)
+    rng = np.random.default_rng(ntri)
+    xyz = rng.uniform(0, 20, (16_000, 3)).astype(np.float32)
+    extent = rng.choice([0.01, 0.5, 6.0], (ntri, 1, 1))
+    tri = rng.uniform(0, 20, (ntri, 1, 3)) + rng.uniform(-1, 1, (ntri, 3, 3)) * extent
+    tri = np.clip(tri, 0, 20).astype(np.float32).reshape(ntri, 9)
+    got = ctx.ion2surf(xyz, tri, R)
+    want = np.asarray(O.ion2surf(xyz, tri, R), np.float32)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
