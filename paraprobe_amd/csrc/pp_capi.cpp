@@ -1658,6 +1658,32 @@ struct Keep {
     }
 };
 
+// Whether a job's k-th neighbour categories are settled from entries (see
+// k_query) rather than one center at a time by windows.  Entries read a task's
+// categories 4 a lane for two centers at once, windows 2 a lane for each
+// center; but every 64 entries read 4 words of each of the task's types again,
+// where 64 more k by windows read nothing.  The line: a task of several
+// types takes entries up to 0.8 steps (of 256 categories or of 64 entries) per
+// step of windows (128 categories of one center), a task of one type up to 1.25;
+// a job's tasks are weighed together.  (200,000 ions, one task, query times with entries and
+// windows: 32 types, C 102, k 300: 2.17 and 0.83 ms; 12 types, C 252, k 64: 0.86 to 0.95
+// of the windows' time, k 200: 1.04 to 1.41; 4 types, C 802, k 10: 0.73 to 0.80; one
+// type, C 52, k 100: 0.98 to 1.07, C 402, k 10: 0.90 to 1.)
+bool knn_entries(const JobPlan &p, int mode, int c16)
+{
+    const int uc = c16 ? 2 : 1;  // centers at a time
+    const int keff = (p.families & PP_FAM_MKNN) ? std::max(p.kmax, 1) : 1;
+    const int64_t ns = (uc * keff + kWave - 1) / kWave;
+    int64_t more = 0;  // by how much entries cost more
+    for (int tk = 0; tk < p.ntasks; ++tk) {
+        const int m = __builtin_popcount(p.task_env[tk]);
+        const int ck = mode == 2 ? (int)(p.task_ck[tk] & 0x7FFFFFFFu) : p.C;
+        const int64_t steps = (ck + 255) / 256 + ns, windows = uc * ((ck + 127) / 128);
+        more += m > 1 ? m * (5 * steps - 4 * windows) : 4 * steps - 5 * windows;
+    }
+    return more <= 0;
+}
+
 // One query launch group: the jobs `ids` (one kernel mode, tiles of T
 // centers) with their device descriptors `base`, as launch chunks, each
 // followed by the reduction of its k-th neighbour categories.  The group's
@@ -1696,11 +1722,13 @@ pp_status launch_group(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std
         return fail(c, PP_ERR_UNSUPPORTED, "histograms too large for LDS (bins x types x tile)");
     std::vector<uint32_t> tile_off(nj + 1, 0);
     std::vector<const JobPlan *> plans(nj);
+    std::vector<int> entries(nj);
     uint32_t total = 0;
     for (int q = 0; q < nj; ++q) {
         tile_off[q] = total;
         total += runs[ids[q]].h_counts[1];
         plans[q] = &runs[ids[q]].plan;
+        entries[q] = mode != 0 && knn_entries(*plans[q], mode, c16) ? 1 : 0;
     }
     tile_off[nj] = total;
     // launch chunks: the k-th neighbour categories of a chunk's tiles must
@@ -1792,6 +1820,7 @@ pp_status launch_group(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std
                 d.kb_tiles = ch.ntl[q];
                 units += (uint32_t)((np + G - 1) / G) * ((ch.ntl[q] + tpu - 1) / tpu);
             }
+            d.k_entries = entries[q];
             hj[k * nj + q] = d;
         }
         huoff[k * (nj + 1) + nj] = units;
@@ -1806,9 +1835,10 @@ pp_status launch_group(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std
     int taskw = 0, entw = 0;
     if (mode != 0) {
         int maxL = 0, keff = 0;
-        for (const JobPlan *p : plans) {
-            maxL = std::max(maxL, p->lmax);
-            keff = std::max(keff, p->kmax);
+        for (int q = 0; q < nj; ++q) {
+            maxL = std::max(maxL, plans[q]->lmax);
+            if (entries[q])
+                keff = std::max(keff, plans[q]->kmax);
         }
         auto room = [&](size_t words) {
             const size_t l = lds + 4 * words;
@@ -1830,9 +1860,11 @@ pp_status launch_group(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std
     if (std::getenv("PP_TRACE_LAUNCH"))
         std::fprintf(stderr,
                      "pp: query mode=%d T=%d c16=%d lds=%zu blocks/CU=%d jobs=%d tiles=%u chunks=%zu "
-                     "maxC=%d maxE=%d maxTrg=%d kmax=%d rows=%d HK=%d\n",
-                     mode, T, c16, lds, nb, nj, total, nch, maxC, maxE, maxTrg, maxK, maxRows,
-                     maxHK);
+                     "maxC=%d maxE=%d maxTrg=%d kmax=%d rows=%d HK=%d taskw=%d entw=%d "
+                     "entries=%d cross=%d\n",
+                     mode, T, c16, lds_all, nb, nj, total, nch, maxC, maxE, maxTrg, maxK, maxRows,
+                     maxHK, taskw, entw, (int)std::count(entries.begin(), entries.end(), 1),
+                     cross ? 1 : 0);
     const bool capture = keep.graph && total > 0;  // (no empty graphs)
     if (capture)
         PP_HIP(c, hipStreamBeginCapture(sl.stream, hipStreamCaptureModeRelaxed));

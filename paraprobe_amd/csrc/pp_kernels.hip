@@ -1574,7 +1574,7 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
             // rows' (free until the next tile) as far as these hold them
             const int ewords = a.entw > 0 ? a.entw : (L.cen - L.rows) / kWaves;
             uint8_t *ent = (uint8_t *)((a.entw > 0 ? s_task + a.taskw : s_rows) + ewords * wid);
-            const bool fits = ne <= 4 * ewords && C <= kEntryCats;
+            const bool fits = J.k_entries != 0 && ne <= 4 * ewords && C <= kEntryCats;
             const int nunit =
                 (want_k || want_1) && kb && fits ? (cnt + UC - 1) / UC : 0;
             for (int u = wid; u < nunit; u += kWaves) {
@@ -1700,7 +1700,8 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
                     if (HY && ((shortm >> h) & 1u))
                         empty_rows(u * UC + h);
             }
-            // k beyond what the entries hold, and categories beyond their bytes
+            // k beyond what the entries hold, categories beyond their bytes,
+            // and jobs for which this is the faster way (knn_entries)
             for (int c = wid; c < cnt && !fits; c += kWaves) {
                 const int hoff = (C16 ? (c >> 1) : c) * (PC ? EC : HK);
                 const int sh = (C16 && (c & 1)) ? 16 : 0;
