@@ -1186,27 +1186,6 @@ int cross_words(bool any, int ntypes) { return any ? (ntypes + 3) & ~3 : 0; }
 
 bool has_cross(const JobRun &r, int mode) { return mode != 1 && r.sym_minor != 0; }
 
-// Workgroups on a CU (6 at most, as its registers allow) of a job in the hybrid
-// mode with cells of Rmax/r, 1/ay of that in y and z, its rows those of
-// symmetric pair counting; 0 in the other modes.
-size_t hybrid_workgroups(const pp_cloud *cl, const JobPlan &p, int T, int r, int ay)
-{
-    if (p.mode != 2 || !(p.families & (PP_FAM_RDF | PP_FAM_RIPK)))
-        return 0;
-    const double w = (double)p.R / r * (1.0 + std::ldexp(1.0, -10));
-    const int nrows = 2 * (int)make_rows(w, w / ay, p.R).size() + 2;
-    int minor = -1;  // the other types that are center and neighbour types
-    for (int s = 0; s < p.ntrg; ++s)
-        minor += p.envoff[p.trg_type[s]] >= 0 && cl->type_count[p.trg_type[s]] > 0;
-    return std::min<size_t>(
-        6, lds_workgroups(query_lds_bytes(T, 1, 2, std::max(p.C, 1), std::max(p.E, 1),
-                                          std::max(p.ntrg, 1), p.kidx_len(), nrows,
-                                          std::max(p.HK, 1),
-                                          (p.E + std::max(minor, 0)) * std::max(p.C, 1) +
-                                              cross_words(minor > 0, type_span(cl)),
-                                          type_span(cl))));
-}
-
 // Symmetric pair counting for a job with pair counts (RDF, RIPK) in the
 // pair-count or the hybrid mode: the center type t with the most ions among the job's center types
 // that are also neighbour types, when t holds at least half of the job's
@@ -1232,124 +1211,190 @@ size_t hybrid_workgroups(const pp_cloud *cl, const JobPlan &p, int T, int r, int
 // Neither of the two is taken where its layout with 32-bit counters, which
 // run_jobs asks of every job, would not fit the LDS: a job that runs without
 // them is not refused for them.
+struct SymPlan {
+    bool on = false;         // symmetric counting
+    uint32_t minor = 0;      // and these types' pairs from t's tiles
+    int type = -1, slot = -1;
+    bool others = false;     // there are candidates of other types than t
+    uint32_t omask[8];
+    std::vector<Row> before, after;
+    size_t wgs = 0;          // workgroups on a CU
+};
+
+// What a job on stencil rows `rows` takes of the two (typed: its candidates are
+// the neighbour types only).
+SymPlan choose_symmetric(const pp_ctx *c, const pp_cloud *cl, const JobPlan &p, bool typed,
+                         bool count_in, int T, const std::vector<Row> &rows)
+{
+    SymPlan y;
+    // (resident workgroups as the register counts allow: 8 in the
+    // pair-count mode, 6 in the hybrid mode)
+    const size_t cap = p.mode == 2 ? 6 : 8;
+    auto bytes = [&](int t, int c16, int nrows, int nminor) {
+        return query_lds_bytes(t, c16, p.mode, std::max(p.C, 1), std::max(p.E, 1),
+                               std::max(p.ntrg, 1), p.kidx_len(), nrows, std::max(p.HK, 1),
+                               (p.E + nminor) * p.C + cross_words(nminor > 0, type_span(cl)),
+                               type_span(cl));
+    };
+    auto wgs = [&](int nrows, int nminor) {
+        return std::min(cap, lds_workgroups(bytes(T, 1, nrows, nminor)));
+    };
+    auto fits = [&](int nrows, int nminor) {
+        return bytes(std::min(T, 8), 0, nrows, nminor) <= c->lds_per_block;
+    };
+    y.wgs = wgs((int)rows.size(), 0);
+    if ((p.mode != 0 && p.mode != 2) || !(p.families & (PP_FAM_RDF | PP_FAM_RIPK)) || cl->n == 0)
+        return y;
+    // the candidates' types: every type of the cloud on the full list, the
+    // neighbour types on a typed list
+    uint32_t cmask[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    uint64_t ncand = 0;
+    for (int t = 0; t < 256; ++t)
+        if (cl->type_count[t] > 0 && (!typed || p.envoff[t] >= 0)) {
+            cmask[t >> 5] |= 1u << (t & 31);
+            ncand += cl->type_count[t];
+        }
+    for (int s = 0; s < p.ntrg; ++s) {
+        const int t = p.trg_type[s];
+        if (p.envoff[t] >= 0 && (y.type < 0 || cl->type_count[t] > cl->type_count[y.type])) {
+            y.type = t;
+            y.slot = s;
+        }
+    }
+    if (y.type < 0 || 2 * cl->type_count[y.type] < ncand)
+        return y;
+    // the row table: own cell, the cells before it (rows of lower z, or of
+    // the same z and lower y, and the own row's part below x), the cells
+    // after it, then every row on the other candidates
+    for (const Row &w : rows) {
+        if (w.dy == 0 && w.dz == 0) {
+            Row b = w, a = w;
+            b.pad = kRowBefore;
+            a.pad = kRowAfter;
+            y.before.push_back(b);
+            y.after.push_back(a);
+        } else if (w.dz < 0 || (w.dz == 0 && w.dy < 0)) {
+            y.before.push_back(w);
+        } else {
+            y.after.push_back(w);
+        }
+    }
+    for (int k = 0; k < 8; ++k) {
+        y.omask[k] = cmask[k] & ~(k == (y.type >> 5) ? 1u << (y.type & 31) : 0u);
+        y.others = y.others || y.omask[k] != 0;
+    }
+    const size_t nsr = 1 + y.before.size() + y.after.size() + (y.others ? rows.size() : 0);
+    if ((int)nsr > kMaxRows || wgs((int)nsr, 0) < y.wgs || !fits((int)nsr, 0))
+        return y;
+    y.on = true;
+    for (int s = 0; s < p.ntrg && y.others && !count_in; ++s)
+        if (s != y.slot && p.envoff[p.trg_type[s]] >= 0 && cl->type_count[p.trg_type[s]] > 0)
+            y.minor |= 1u << s;
+    const int nminor = __builtin_popcount(y.minor);
+    if (y.minor && (wgs((int)nsr, nminor) < y.wgs || !fits((int)nsr, nminor)))
+        y.minor = 0;
+    return y;
+}
+
 pp_status plan_symmetric(pp_ctx *c, Slot &sl, pp_cloud *cl, JobRun &r)
 {
     r.sym_slot = -1;
     r.sym_minor = 0;
     r.srows.clear();
     const JobPlan &p = r.plan;
-    if ((p.mode != 0 && p.mode != 2) || !(p.families & (PP_FAM_RDF | PP_FAM_RIPK)) ||
-        cl->n == 0 || sl.fixed)
+    if (sl.fixed)
         return PP_OK;
-    // the candidates' types: every type of the cloud on the full list, the
-    // neighbour types on a typed list
-    uint32_t cmask[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    uint64_t ncand = 0;
-    for (int t = 0; t < 256; ++t)
-        if (cl->type_count[t] > 0 && (r.cand == r.cl || p.envoff[t] >= 0)) {
-            cmask[t >> 5] |= 1u << (t & 31);
-            ncand += cl->type_count[t];
-        }
-    int best = -1, bslot = -1;
-    for (int s = 0; s < p.ntrg; ++s) {
-        const int t = p.trg_type[s];
-        if (p.envoff[t] >= 0 && (best < 0 || cl->type_count[t] > cl->type_count[best])) {
-            best = t;
-            bslot = s;
-        }
-    }
-    if (best < 0 || 2 * cl->type_count[best] < ncand)
+    const SymPlan y = choose_symmetric(c, cl, p, r.cand != r.cl, r.count_in, r.T_req, r.rows);
+    if (!y.on)
         return PP_OK;
-    // the row table: own cell, the cells before it (rows of lower z, or of
-    // the same z and lower y, and the own row's part below x), the cells
-    // after it, then every row on the other candidates
-    std::vector<Row> before, after;
-    for (const Row &w : r.rows) {
-        if (w.dy == 0 && w.dz == 0) {
-            Row b = w, a = w;
-            b.pad = kRowBefore;
-            a.pad = kRowAfter;
-            before.push_back(b);
-            after.push_back(a);
-        } else if (w.dz < 0 || (w.dz == 0 && w.dy < 0)) {
-            before.push_back(w);
-        } else {
-            after.push_back(w);
-        }
-    }
-    uint32_t omask[8];
-    bool others = false;
-    for (int k = 0; k < 8; ++k) {
-        omask[k] = cmask[k] & ~(k == (best >> 5) ? 1u << (best & 31) : 0u);
-        others = others || omask[k] != 0;
-    }
-    const size_t nsr = 1 + before.size() + after.size() + (others ? r.rows.size() : 0);
-    if ((int)nsr > kMaxRows)
-        return PP_OK;
-    uint32_t minor = 0;
-    {
-        // (resident workgroups as the register counts allow: 8 in the
-        // pair-count mode, 6 in the hybrid mode)
-        const size_t cap = p.mode == 2 ? 6 : 8;
-        auto bytes = [&](int T, int c16, int nrows, int nminor) {
-            return query_lds_bytes(T, c16, p.mode, std::max(p.C, 1), std::max(p.E, 1),
-                                   std::max(p.ntrg, 1), p.kidx_len(), nrows, std::max(p.HK, 1),
-                                   (p.E + nminor) * p.C + cross_words(nminor > 0, type_span(cl)),
-                                   type_span(cl));
-        };
-        auto wgs = [&](int nrows, int nminor) {
-            return std::min(cap, lds_workgroups(bytes(r.T_req, 1, nrows, nminor)));
-        };
-        auto fits = [&](int nrows, int nminor) {
-            return bytes(std::min(r.T_req, 8), 0, nrows, nminor) <= c->lds_per_block;
-        };
-        const size_t base = wgs((int)r.rows.size(), 0);
-        if (wgs((int)nsr, 0) < base || !fits((int)nsr, 0))
-            return PP_OK;
-        for (int s = 0; s < p.ntrg && others && !r.count_in; ++s)
-            if (s != bslot && p.envoff[p.trg_type[s]] >= 0 &&
-                cl->type_count[p.trg_type[s]] > 0)
-                minor |= 1u << s;
-        const int nminor = __builtin_popcount(minor);
-        if (minor && (wgs((int)nsr, nminor) < base || !fits((int)nsr, nminor)))
-            minor = 0;
-    }
     uint32_t smask[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    smask[best >> 5] = 1u << (best & 31);
+    smask[y.type >> 5] = 1u << (y.type & 31);
     const CellList *S = nullptr, *O = nullptr;
     pp_status st = get_sublist(c, sl, cl, r.cl, smask, S, 1);
     if (st != PP_OK)
         return st;
     if (S == r.cl || !S->w_s2)
         return PP_OK;
-    if (others) {
-        st = get_sublist(c, sl, cl, r.cl, omask, O, 0);
+    if (y.others) {
+        st = get_sublist(c, sl, cl, r.cl, y.omask, O, 0);
         if (st != PP_OK)
             return st;
         if (O == r.cl)
             return PP_OK;
     }
     r.srows.push_back(Row{0, 0, 0, 0});
-    r.srows.insert(r.srows.end(), before.begin(), before.end());
-    r.srows.insert(r.srows.end(), after.begin(), after.end());
-    r.s_nb1 = 1 + (int)before.size();
-    r.s_ns = r.s_nb1 + (int)after.size();
-    if (others)
+    r.srows.insert(r.srows.end(), y.before.begin(), y.before.end());
+    r.srows.insert(r.srows.end(), y.after.begin(), y.after.end());
+    r.s_nb1 = 1 + (int)y.before.size();
+    r.s_ns = r.s_nb1 + (int)y.after.size();
+    if (y.others)
         r.srows.insert(r.srows.end(), r.rows.begin(), r.rows.end());
     r.symS = S;
     r.symO = O;
-    r.sym_slot = bslot;
-    r.sym_type = best;
-    r.sym_minor = minor;
+    r.sym_slot = y.slot;
+    r.sym_type = y.type;
+    r.sym_minor = y.minor;
     // t's kNN range (d2 <= its threshold), widened like the in-ball reach
     r.kreach = -1.0;
-    if (!p.kinfo.empty() && p.kinfo[2 * best] >= 0) {
+    if (!p.kinfo.empty() && p.kinfo[2 * y.type] >= 0) {
         float kthr;
-        std::memcpy(&kthr, &p.kinfo[2 * best + 1], 4);
+        std::memcpy(&kthr, &p.kinfo[2 * y.type + 1], 4);
         if (kthr >= 0.0f)
             r.kreach = std::sqrt((double)kthr) * (1.0 + std::ldexp(1.0, -12)) + 1e-4 * r.cl->g.w;
     }
     return PP_OK;
+}
+
+// A job's candidates are its neighbour types' ions only, a list of their own,
+// when these are a minority.
+bool typed_candidates(const pp_cloud *cl, const JobPlan &p)
+{
+    uint64_t inenv = 0;
+    for (int e = 0; e < p.E; ++e)
+        inenv += cl->type_count[p.env_type[e]];
+    return cl->n > 0 && (double)inenv < 0.8 * (double)cl->n;
+}
+
+// Whether the kernel counts a job's in-ball pairs.  The total needs no count
+// of its own where the RDF pair counts give it, every ion type of the cloud
+// being a neighbour type of the job, nor where there is none to give: a typed
+// list holds the neighbour types only (pairs_inball is -1 then).  The count is
+// a ballot and a 64-bit add per center and wavefront step.
+bool counts_inball(const pp_cloud *cl, const JobPlan &p, bool typed)
+{
+    if (typed)
+        return false;
+    if (!(p.families & (PP_FAM_RDF | PP_FAM_RIPK)))
+        return true;
+    for (int t = 0; t < 256; ++t)
+        if (cl->type_count[t] > 0 && p.envoff[t] < 0)
+            return true;
+    return false;
+}
+
+// In the hybrid mode with pair counts, where the density rule takes cells of
+// Rmax/2 by Rmax/4: cubes of Rmax/3 instead, whose row table is shorter and
+// whose evaluations cost 2 % more, where the shorter table leaves more
+// workgroups on a CU, or as many and symmetric or cross-type counting that the
+// longer one has no room for -- and takes neither of these away.  (20M ions, R 5
+// nm, query kernel: k to 10 120.5 and 123.2 ms, k to 100, with six workgroups and
+// five, 128.9 and 137.7.  300,000 ions, 36 per nm^3: R 5, three types, 600 bins, k to
+// 100, with cross-type rows only in cubes, 2.79 and 3.24 ms; R 4.2, 1,000 bins, k to 5,
+// five workgroups without symmetric counting against four with it, 2.86 and
+// 2.41: not taken.)
+bool cubes_of_third(const pp_ctx *c, const pp_cloud *cl, const JobPlan &p, int T)
+{
+    if (p.mode != 2 || !(p.families & (PP_FAM_RDF | PP_FAM_RIPK)))
+        return false;
+    const bool typed = typed_candidates(cl, p), count_in = counts_inball(cl, p, typed);
+    auto plan = [&](int r, int ay) {
+        const double w = (double)p.R / r * (1.0 + std::ldexp(1.0, -10));
+        return choose_symmetric(c, cl, p, typed, count_in, T, make_rows(w, w / ay, p.R));
+    };
+    const SymPlan cube = plan(3, 1), longer = plan(2, 2);
+    const int gain = (cube.on ? 1 : 0) + (cube.minor ? 1 : 0) - (longer.on ? 1 : 0) -
+                     (longer.minor ? 1 : 0);
+    return gain >= 0 && (gain > 0 ? cube.wgs >= longer.wgs : cube.wgs > longer.wgs);
 }
 
 void compose_outputs(const JobRun &r, const std::vector<unsigned long long> &P,
@@ -2106,14 +2151,9 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
         // the rule's cells of Rmax/4 and Rmax/2 are taken twice as long
         // along x in the lists jobs build for themselves (Rmax/2 by Rmax/4,
         // Rmax by Rmax/2): the same stencil rows, each of half as many cells.
-        // Cubes of Rmax/3 instead of Rmax/2 by Rmax/4, whose evaluations cost
-        // 2 % more, where their shorter row table leaves more workgroups on a
-        // CU (20M ions, R 5 nm: k to 10 120.5 and 123.2 ms of query kernel, k
-        // to 100, with five and six workgroups, 137.7 and 128.9)
         if (by_rule && tuneAY <= 0 && jAY <= 0 && (p.r == 4 || p.r == 2) &&
             !clouds[i]->resident) {
-            if (p.r == 4 && hybrid_workgroups(clouds[i], p, jT, 3, 1) >
-                                hybrid_workgroups(clouds[i], p, jT, 2, 2)) {
+            if (p.r == 4 && cubes_of_third(c, clouds[i], p, jT)) {
                 p.r = 3;
             } else {
                 p.r /= 2;
@@ -2143,33 +2183,17 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
             // only the neighbour types are candidates when they are a minority
             const JobPlan &p = runs[i].plan;
             const pp_cloud *cl = clouds[i];
-            uint64_t inenv = 0;
             uint32_t mask[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-            for (int e = 0; e < p.E; ++e) {
-                inenv += cl->type_count[p.env_type[e]];
+            for (int e = 0; e < p.E; ++e)
                 mask[p.env_type[e] >> 5] |= 1u << (p.env_type[e] & 31);
-            }
-            if (cl->n > 0 && (double)inenv < 0.8 * (double)cl->n) {
+            if (typed_candidates(cl, p)) {
                 st = get_sublist(c, sl, const_cast<pp_cloud *>(cl), runs[i].cl, mask,
                                  runs[i].cand);
                 if (st != PP_OK)
                     return st;
             }
         }
-        {
-            // the in-ball total needs no count of its own where the RDF pair
-            // counts give it, every ion type of the cloud being a neighbour
-            // type of the job, nor where there is none to give: a typed list
-            // holds the neighbour types only (pairs_inball is -1 below).  The
-            // count is a ballot and a 64-bit add per center and wavefront step.
-            const JobPlan &p = runs[i].plan;
-            const bool typed = runs[i].cand != runs[i].cl;
-            bool all_env = !typed;
-            for (int t = 0; t < 256 && all_env; ++t)
-                if (clouds[i]->type_count[t] > 0 && p.envoff[t] < 0)
-                    all_env = false;
-            runs[i].count_in = !typed && !(all_env && (p.families & (PP_FAM_RDF | PP_FAM_RIPK)));
-        }
+        runs[i].count_in = counts_inball(clouds[i], runs[i].plan, runs[i].cand != runs[i].cl);
         runs[i].rows = make_rows(runs[i].cl->g.w, runs[i].cl->g.wyz, runs[i].plan.R);
         if ((int)runs[i].rows.size() > kMaxRows)
             return fail(c, PP_ERR_UNSUPPORTED, "stencil too large (cell width far below Rmax)");
