@@ -839,7 +839,8 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
 
         if (pkey != cur || (!done && pending > 0x7FFFFFFFull)) {
             if (cur >= 0) {
-                // flush the accumulated pair counts and statistics
+                // flush the accumulated pair counts and, behind a job's last
+                // tile here, its statistics
                 const CJobDev &P0 = jobs[cur / kMaxTrg];
                 const int n = P0.E * P0.C;
                 if (P0.families & (FAM_RDF | FAM_RIPK)) {
@@ -867,12 +868,17 @@ __global__ __launch_bounds__(kBlock, (T == 8 && MODE == 0) ? 8 : (T == 8 && MODE
                         }
                     }
                 }
-                if (lane == 0 && inball)
-                    atomicAdd(&P0.stats[0], inball);
-                if (tid == 0 && cand)
-                    atomicAdd(&P0.stats[1], cand);
-                inball = 0;
-                cand = 0;
+                // (two words that every workgroup of the job adds to: with a
+                // flush per center type, few-center types cost their kernel
+                // more than their tiles did)
+                if (job != cur / kMaxTrg) {
+                    if (lane == 0 && inball)
+                        atomicAdd(&P0.stats[0], inball);
+                    if (tid == 0 && cand)
+                        atomicAdd(&P0.stats[1], cand);
+                    inball = 0;
+                    cand = 0;
+                }
                 pending = 0;
                 __syncthreads();
             }
