@@ -218,8 +218,10 @@ hipError_t launch_npcorr(const NpcArgs &a, hipStream_t s);
 
 // The fixed scratch of the no-allocation entry point (pp_noalloc.hip): the
 // device address of this device's copy (looked up once per device) and its
-// size.
-constexpr size_t kNoAllocBytes = size_t(256) << 20;
+// size.  Above 256 MiB what the preparation's lists may take beyond the room
+// kept for them (layout_prep): 384 bytes per center type where a type has less
+// than a block of ions, 16 of its PrepSeg, and their alignment, 14.3 KiB for 32.
+constexpr size_t kNoAllocBytes = (size_t(256) << 20) + (size_t(16) << 10);
 constexpr int kMaxDevices = 64;
 hipError_t noalloc_scratch(int device, void **ptr, size_t *bytes);
 
