@@ -1902,14 +1902,20 @@ pp_status launch_group(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std
     PP_HIP(c, query_max_blocks_per_cu(T, c16, mode, lds_all, &nb));
     if (nb < 1)
         nb = 1;
-    if (std::getenv("PP_TRACE_LAUNCH"))
+    if (std::getenv("PP_TRACE_LAUNCH")) {
+        // jobs whose k-th neighbours are settled from entries, as the kernel decides
+        const int ew = entw > 0 ? entw : query_row_words(maxRows, mode) / kWaves;
+        int ent = 0;
+        for (int q = 0; q < nj; ++q)
+            ent += entries[q] && plans[q]->nplanes() > 0 && plans[q]->C <= kEntryCats &&
+                   (c16 ? 2 : 1) * std::max(plans[q]->kmax, 1) <= 4 * ew;
         std::fprintf(stderr,
                      "pp: query mode=%d T=%d c16=%d lds=%zu blocks/CU=%d jobs=%d tiles=%u chunks=%zu "
                      "maxC=%d maxE=%d maxTrg=%d kmax=%d rows=%d HK=%d taskw=%d entw=%d "
                      "entries=%d cross=%d\n",
                      mode, T, c16, lds_all, nb, nj, total, nch, maxC, maxE, maxTrg, maxK, maxRows,
-                     maxHK, taskw, entw, (int)std::count(entries.begin(), entries.end(), 1),
-                     cross ? 1 : 0);
+                     maxHK, taskw, entw, ent, cross ? 1 : 0);
+    }
     const bool capture = keep.graph && total > 0;  // (no empty graphs)
     if (capture)
         PP_HIP(c, hipStreamBeginCapture(sl.stream, hipStreamCaptureModeRelaxed));
