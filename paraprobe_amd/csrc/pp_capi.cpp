@@ -904,11 +904,12 @@ void layout_prep(PrepArena &a, Carver &m, bool fixed)
     a.js = m.take<PrepJobStat>((size_t)std::max(a.njobs, 1));
 }
 
-// The part of the arena that is uploaded (the run's tables follow it)
+// The part of the arena that is uploaded, the segments last (a rerun's few
+// are all that goes up of them; the run's tables follow their room)
 void layout_prep_upload(PrepArena &a, Carver &m)
 {
-    a.segs = m.take<PrepSeg>((size_t)std::max(a.nseg, 1));
     a.jseg = m.take<int32_t>((size_t)a.njobs + 1);
+    a.segs = m.take<PrepSeg>((size_t)std::max(a.nseg, 1));
 }
 
 // Bytes of one job's share of a run's scratch (admission control).
@@ -961,22 +962,32 @@ void stage_tables(const JobRun &r, uint32_t *h)
 // selected by the considered rule, or, for the full-range rerun, by the
 // job's rerun marks.  Reads back each job's center and tile counts and its
 // stencil candidate bound; the lists stay valid until the next prep_run.
-// tables: the run's tables, uploaded to tables_dev (behind the arena's segment
-// list) in the same copy, or null.
+// tables: the host image of the arena's upload with the run's tables behind the
+// room for the segment list, which goes up in the same copy, or null.
 pp_status prep_run(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std::vector<int> &ids,
-                   PrepArena &a, bool rerun, const std::vector<uint32_t> *tables,
-                   const uint32_t *tables_dev)
+                   PrepArena &a, bool rerun, std::vector<char> *tables)
 {
     const int nj = (int)ids.size();
     if (nj == 0)
         return PP_OK;
-    std::vector<PrepSeg> segs;
-    std::vector<int32_t> jseg(nj + 1, 0);
+    int nseg = 0;
+    for (int q = 0; q < nj; ++q)
+        nseg += runs[ids[q]].plan.ntrg;
+    if (nseg > a.nseg || nj > a.njobs)
+        return fail(c, PP_ERR_HIP, "internal: preparation larger than its arena");
+    // the host image of the upload; the lists are written in place
+    char *const up0 = (char *)a.jseg;
+    const size_t seg_off = (size_t)((const char *)a.segs - up0);
+    std::vector<char> own(tables ? 0 : seg_off + (size_t)nseg * sizeof(PrepSeg));
+    std::vector<char> &up = tables ? *tables : own;
+    int32_t *const jseg = (int32_t *)up.data();
+    PrepSeg *const segs = (PrepSeg *)(up.data() + seg_off);
+    int ns = 0;
     uint64_t E = 0, Ec = 0, nc = 0, jblocks = 0;
     for (int q = 0; q < nj; ++q) {
         JobRun &r = runs[ids[q]];
         const JobPlan &p = r.plan;
-        jseg[q] = (int32_t)segs.size();
+        jseg[q] = ns;
         for (int slot = 0; slot < p.ntrg; ++slot) {
             PrepSeg g{};
             g.pos = r.cl->pos;
@@ -997,7 +1008,7 @@ pp_status prep_run(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std::ve
             g.slot = slot;
             g.T = r.T_req;
             g.job = q;
-            segs.push_back(g);
+            segs[ns++] = g;
             E += prep_pad(r.cloud->n);
             Ec += prep_pad(r.ncells);
             nc += r.ncells;
@@ -1005,25 +1016,14 @@ pp_status prep_run(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std::ve
         if (p.ntrg > 0)
             jblocks += prep_pad(r.cloud->n) / kPrepTile;
     }
-    jseg[nj] = (int32_t)segs.size();
-    if (E > a.E || Ec > a.Ec || nc > a.nc || (int)segs.size() > a.nseg || nj > a.njobs)
+    jseg[nj] = ns;
+    if (E > a.E || Ec > a.Ec || nc > a.nc)
         return fail(c, PP_ERR_HIP, "internal: preparation larger than its arena");
     hipStream_t s = sl.stream;
-    char *const up0 = (char *)a.segs;
-    std::vector<char> up(tables ? (size_t)((const char *)tables_dev - up0) + tables->size() * 4
-                                : (size_t)((const char *)a.jseg - up0) + jseg.size() * 4);
-    auto stage = [&](const void *dev, const void *src, size_t bytes) {
-        if (bytes)
-            std::memcpy(up.data() + ((const char *)dev - up0), src, bytes);
-    };
-    stage(a.segs, segs.data(), segs.size() * sizeof(PrepSeg));
-    stage(a.jseg, jseg.data(), jseg.size() * 4);
-    if (tables)
-        stage(tables_dev, tables->data(), tables->size() * 4);
     PP_HIP(c, hipMemcpyAsync(up0, up.data(), up.size(), hipMemcpyHostToDevice, s));
     PrepLaunch L;
     L.segs = a.segs;
-    L.nseg = (int)segs.size();
+    L.nseg = nseg;
     L.jseg = a.jseg;
     L.njobs = nj;
     L.E = E;
@@ -2281,17 +2281,18 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
     carve(m, out0, out1);
     const size_t out_bytes = (size_t)(out1 - out0);
     {
-        std::vector<uint32_t> h(tables_words, 0u);
-        size_t o = 0;
+        const size_t head = (size_t)((const char *)tables_dev - (const char *)pa.jseg);
+        std::vector<char> up(head + 4 * tables_words, 0);
+        size_t o = head;
         for (int i = 0; i < njobs; ++i) {
-            stage_tables(runs[i], h.data() + o);
-            o += runs[i].tables_words;
+            stage_tables(runs[i], (uint32_t *)(up.data() + o));
+            o += 4 * runs[i].tables_words;
         }
         PP_HIP(c, hipMemsetAsync(out0, 0, (size_t)(clear1 - out0), sl.stream));
         std::vector<int> all(njobs);
         for (int i = 0; i < njobs; ++i)
             all[i] = i;
-        st = prep_run(c, sl, runs, all, pa, false, &h, tables_dev);
+        st = prep_run(c, sl, runs, all, pa, false, &up);
         if (st != PP_OK)
             return st;
     }
@@ -2418,7 +2419,7 @@ pp_status run_jobs(pp_ctx *c, Slot &sl, int njobs, const pp_cloud *const *clouds
                            c->lds_per_block)
                     r.T_req /= 2;
             }
-            st = prep_run(c, sl, runs, hy, pa, true, nullptr, nullptr);
+            st = prep_run(c, sl, runs, hy, pa, true, nullptr);
             if (st != PP_OK)
                 return st;
             std::vector<int> ids1, modes1;
