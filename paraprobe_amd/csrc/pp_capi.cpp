@@ -898,6 +898,7 @@ void layout_prep(PrepArena &a, Carver &m, bool fixed)
     a.l.boff = m.take<uint32_t>(w.boff);
     a.l.tpre = m.take<uint32_t>(w.tpre);
     a.l.toff = m.take<uint32_t>(w.toff);
+    a.l.seg = m.take<uint32_t>(w.seg);
     m.off = std::max(m.off, room.off);
     a.centers = m.take<uint32_t>(a.nion + 1);
     a.tiles = m.take<Tile>(a.nion + 1);  // at most one tile per center
@@ -1028,6 +1029,7 @@ pp_status prep_run(pp_ctx *c, Slot &sl, std::vector<JobRun> &runs, const std::ve
     L.njobs = nj;
     L.E = E;
     L.Ec = Ec;
+    L.nc = nc;
     L.jblocks = (uint32_t)jblocks;
     L.l = a.l;
     L.centers = a.centers;

@@ -87,13 +87,14 @@ struct PrepSeg {
 };
 // The run's temporary lists: a bit per element of the ion space, the centers
 // before each 64 of them in their block, the centers before each block (and
-// the total); the tiles before each cell in its block and before each block.
+// the total); the tiles before each cell in its block and before each block; the
+// segment of each block of the ion space, then of the cell space.
 struct PrepLists {
     uint64_t *bits;
-    uint32_t *wpos, *boff, *tpre, *toff;
+    uint32_t *wpos, *boff, *tpre, *toff, *seg;
 };
 struct PrepWords {
-    size_t bits, wpos, boff, tpre, toff;  // sizes in 4-byte words
+    size_t bits, wpos, boff, tpre, toff, seg;  // sizes in 4-byte words
 };
 PrepWords prep_words(uint64_t E, uint64_t Ec, uint64_t nc);  // nc: cells of all segments
 // Per job: its centers [center0, center0 + centers) of the run's center list,
@@ -108,6 +109,7 @@ struct PrepLaunch {
     const int32_t *jseg;       // device [njobs + 1]: job j's segments [jseg[j], jseg[j + 1])
     int njobs;
     uint64_t E, Ec;            // sizes of the ion and cell spaces (multiples of kPrepTile)
+    uint64_t nc;               // cells of all segments
     uint32_t jblocks;          // blocks of kPrepTile ions, each job's ions counted once
     PrepLists l;
     uint32_t *centers;         // the run's center list (job-local sorted ion indices)
@@ -219,8 +221,8 @@ hipError_t launch_npcorr(const NpcArgs &a, hipStream_t s);
 // The fixed scratch of the no-allocation entry point (pp_noalloc.hip): the
 // device address of this device's copy (looked up once per device) and its
 // size.  Above 256 MiB what the preparation's lists may take beyond the room
-// kept for them (layout_prep): 384 bytes per center type where a type has less
-// than a block of ions, 16 of its PrepSeg, and their alignment, 14.3 KiB for 32.
+// kept for them (layout_prep): 392 bytes per center type where a type has less
+// than a block of ions, 16 of its PrepSeg, and their alignment, 14.8 KiB for 32.
 constexpr size_t kNoAllocBytes = (size_t(256) << 20) + (size_t(16) << 10);
 constexpr int kMaxDevices = 64;
 hipError_t noalloc_scratch(int device, void **ptr, size_t *bytes);

@@ -23,7 +23,10 @@
 // again), and for small runs the number of launches, 5 instead of 12.  A
 // whole call, before and after: 20,000 ions with three center types 303 and
 // 283 us, a batch of 24 jobs of 50,000 to 2,000,000 ions 7.73 and 7.20 ms, 100
-// million ions with one center type 423 and 415 ms.
+// million ions with one center type 423 and 415 ms.  A run of many small jobs is
+// bound by its blocks' first loads: the segment of a block is looked up in a list
+// that the first launch writes (bisecting the segments in every block took
+// 0.65 ms for 27,000 segments of 27 cells).
 #include "pp_launch.h"
 
 namespace pp {
@@ -66,7 +69,8 @@ __device__ inline uint32_t center_pos(const PrepLists &l, uint64_t e)
 }
 
 // One block per kPrepTile ions of a job, for all of the job's segments.
-__global__ __launch_bounds__(kPrepBlock) void k_pflags(const PrepSeg *__restrict__ segs,
+__global__ __launch_bounds__(kPrepBlock) void k_pflags(const PrepSeg *__restrict__ segs, int nseg,
+                                                        uint32_t nion,
                                                         const int32_t *__restrict__ jseg, int njobs,
                                                         PrepLists l, PrepJobStat *__restrict__ js)
 {
@@ -75,6 +79,17 @@ __global__ __launch_bounds__(kPrepBlock) void k_pflags(const PrepSeg *__restrict
     if (blockIdx.x == 0)
         for (int k = threadIdx.x; k < njobs; k += kPrepBlock)
             js[k].maxcand = 0u;
+    // the segment of each block of the ion space and of the cell space
+    for (int q = blockIdx.x; q < nseg; q += gridDim.x) {
+        const PrepSeg &Q = segs[q];
+        const uint64_t ib = Q.ion0 / kPrepTile, cb = nion + Q.cell0 / kPrepTile;
+        const uint32_t in = (uint32_t)(((uint64_t)Q.n + kPrepTile - 1) / kPrepTile);
+        const uint32_t cn = (uint32_t)(((uint64_t)Q.nc + kPrepTile - 1) / kPrepTile);
+        for (uint32_t k = threadIdx.x; k < in; k += kPrepBlock)
+            l.seg[ib + k] = (uint32_t)q;
+        for (uint32_t k = threadIdx.x; k < cn; k += kPrepBlock)
+            l.seg[cb + k] = (uint32_t)q;
+    }
     // (a job without segments starts where the next one does and owns no block)
     const int j = find_last(blockIdx.x, njobs, [&](int k) {
         return jseg[k] < jseg[njobs] ? (uint64_t)segs[jseg[k]].jblk0 : ~0ull; }, &s_q);
@@ -171,16 +186,14 @@ __global__ __launch_bounds__(1024) void k_pscan(uint32_t *__restrict__ v, uint32
 // sorted ion indices); the others: the tiles per cell of one block of the
 // cell space, as their prefix in the block and the block's total.
 __global__ __launch_bounds__(kPrepBlock) void k_pcompact(const PrepSeg *__restrict__ segs,
-                                                          int nseg, uint32_t nion, PrepLists l,
+                                                          uint32_t nion, PrepLists l,
                                                           uint32_t *__restrict__ centers)
 {
-    __shared__ int s_q;
     __shared__ uint32_t s_w[kPrepBlock / 64];
     const int lane = threadIdx.x & 63, wid = threadIdx.x / 64;
     if (blockIdx.x < nion) {
         const uint64_t e0 = (uint64_t)blockIdx.x * kPrepTile;
-        const int q = find_last(e0, nseg, [&](int k) { return segs[k].ion0; }, &s_q);
-        const uint32_t i0 = (uint32_t)(e0 - segs[q].ion0), off = l.boff[blockIdx.x];
+        const uint32_t i0 = (uint32_t)(e0 - segs[l.seg[blockIdx.x]].ion0), off = l.boff[blockIdx.x];
         for (int k = 0; k < kPrepItems; ++k) {
             const uint64_t w = e0 / 64 + (uint64_t)(k * (kPrepBlock / 64) + wid);
             const uint64_t m = l.bits[w];
@@ -193,8 +206,7 @@ __global__ __launch_bounds__(kPrepBlock) void k_pcompact(const PrepSeg *__restri
     }
     const uint32_t cb = blockIdx.x - nion;
     const uint64_t e0 = (uint64_t)cb * kPrepTile;
-    const int q = find_last(e0, nseg, [&](int k) { return segs[k].cell0; }, &s_q);
-    const PrepSeg S = segs[q];
+    const PrepSeg S = segs[l.seg[blockIdx.x]];
     const uint64_t c0 = e0 - S.cell0 + (uint64_t)threadIdx.x * kPrepItems;
     uint32_t cnt[kPrepItems], tot = 0;
     uint32_t lo = c0 < S.nc ? center_pos(l, S.ion0 + S.cellstart[c0]) : 0u;
@@ -250,14 +262,13 @@ __device__ inline uint32_t row_count(const Row &rw, int cx, int cy, int cz, cons
 // candidate count (a bound on any center's neighbour count); the first block
 // also writes each job's parts of the run's lists.
 __global__ __launch_bounds__(kPrepBlock) void k_ptilewrite(const PrepSeg *__restrict__ segs,
-                                                            int nseg,
+                                                            uint32_t nion, uint32_t ncell,
+                                                            uint32_t per,
                                                             const int32_t *__restrict__ jseg,
                                                             int njobs, PrepLists l,
                                                             Tile *__restrict__ tiles,
                                                             PrepJobStat *__restrict__ js)
 {
-    __shared__ int s_q;
-    const uint64_t b0 = (uint64_t)blockIdx.x * kPrepBlock;
     if (blockIdx.x == 0)
         for (int j = threadIdx.x; j < njobs; j += kPrepBlock) {
             const int a = jseg[j], b = jseg[j + 1];
@@ -276,43 +287,50 @@ __global__ __launch_bounds__(kPrepBlock) void k_ptilewrite(const PrepSeg *__rest
             js[j].tile0 = t0;
             js[j].tiles = t1 - t0;
         }
-    const int q = find_last(b0, nseg, [&](int k) { return segs[k].cell0; }, &s_q);
-    const PrepSeg S = segs[q];  // by value: kept in registers, not re-read
-    const uint64_t e = b0 + threadIdx.x;
-    const uint64_t c = e - S.cell0;
-    // every lane stays to the wave's reduction below (no early return)
-    uint32_t tot = 0;
-    if (c < S.nc) {
-        const uint32_t lo = center_pos(l, S.ion0 + S.cellstart[c]),
-                       hi = center_pos(l, S.ion0 + S.cellstart[c + 1]);
-        if (hi > lo) {
-            const uint32_t T = (uint32_t)S.T, cnt = hi - lo;
-            const uint32_t t0 = l.toff[e / kPrepTile] + l.tpre[S.tp0 + c];
-            for (uint32_t m = 0; m * T < cnt; ++m) {
-                Tile t;
-                t.key = (uint32_t)c;
-                t.first = lo + m * T;
-                const uint32_t left = cnt - m * T;
-                t.count = (uint16_t)(left < T ? left : T);
-                t.job = (uint16_t)S.job;
-                t.pad = (uint32_t)S.slot;
-                tiles[t0 + m] = t;
-            }
-            const int cx = (int)(c % (uint64_t)S.g.nx);
-            const int cy = (int)((c / (uint64_t)S.g.nx) % (uint64_t)S.g.ny);
-            const int cz = (int)(c / ((uint64_t)S.g.nx * (uint64_t)S.g.ny));
+    // block blockIdx.x / per of the cell space, every per-th kPrepBlock of its cells
+    const uint32_t cb = blockIdx.x / per;
+    if (cb >= ncell)
+        return;
+    const PrepSeg S = segs[l.seg[nion + cb]];  // by value: kept in registers, not re-read
+    for (uint32_t it = blockIdx.x % per; it < (uint32_t)kPrepItems; it += per) {
+        const uint64_t cw = (uint64_t)cb * kPrepTile + it * (uint32_t)kPrepBlock - S.cell0;
+        if (cw >= S.nc)
+            return;
+        const uint64_t c = cw + threadIdx.x;
+        // every lane stays to the wave's reduction below
+        uint32_t tot = 0;
+        if (c < S.nc) {
+            const uint32_t lo = center_pos(l, S.ion0 + S.cellstart[c]),
+                           hi = center_pos(l, S.ion0 + S.cellstart[c + 1]);
+            if (hi > lo) {
+                const uint32_t T = (uint32_t)S.T, cnt = hi - lo;
+                const uint32_t t0 = l.toff[cb] + l.tpre[S.tp0 + c];
+                for (uint32_t m = 0; m * T < cnt; ++m) {
+                    Tile t;
+                    t.key = (uint32_t)c;
+                    t.first = lo + m * T;
+                    const uint32_t left = cnt - m * T;
+                    t.count = (uint16_t)(left < T ? left : T);
+                    t.job = (uint16_t)S.job;
+                    t.pad = (uint32_t)S.slot;
+                    tiles[t0 + m] = t;
+                }
+                const int cx = (int)(c % (uint64_t)S.g.nx);
+                const int cy = (int)((c / (uint64_t)S.g.nx) % (uint64_t)S.g.ny);
+                const int cz = (int)(c / ((uint64_t)S.g.nx * (uint64_t)S.g.ny));
 #pragma unroll 4
-            for (int r = 0; r < S.nrows; ++r)
-                tot += row_count(S.rows[r], cx, cy, cz, S.g, S.cellstart);
+                for (int r = 0; r < S.nrows; ++r)
+                    tot += row_count(S.rows[r], cx, cy, cz, S.g, S.cellstart);
+            }
         }
+        // one atomic per wavefront (a block's cells belong to one job)
+        for (int d = 32; d > 0; d >>= 1) {
+            const uint32_t o = (uint32_t)__shfl_xor((int)tot, d, 64);
+            tot = o > tot ? o : tot;
+        }
+        if ((threadIdx.x & 63) == 0 && tot > 0)
+            atomicMax(&js[S.job].maxcand, tot);
     }
-    // one atomic per wavefront (a block's cells belong to one job)
-    for (int d = 32; d > 0; d >>= 1) {
-        const uint32_t o = (uint32_t)__shfl_xor((int)tot, d, 64);
-        tot = o > tot ? o : tot;
-    }
-    if ((threadIdx.x & 63) == 0 && tot > 0)
-        atomicMax(&js[S.job].maxcand, tot);
 }
 
 } // namespace
@@ -325,6 +343,7 @@ PrepWords prep_words(uint64_t E, uint64_t Ec, uint64_t nc)
     w.boff = E / kPrepTile + 1;
     w.tpre = nc;
     w.toff = Ec / kPrepTile + 1;
+    w.seg = E / kPrepTile + Ec / kPrepTile;
     return w;
 }
 
@@ -334,22 +353,28 @@ hipError_t launch_prep(const PrepLaunch &p, hipStream_t s)
         return hipSuccess;
     const uint32_t nion = (uint32_t)(p.E / kPrepTile), ncell = (uint32_t)(p.Ec / kPrepTile);
     hipError_t e;
-    hipLaunchKernelGGL(k_pflags, dim3(p.jblocks ? p.jblocks : 1), dim3(kPrepBlock), 0, s, p.segs, p.jseg, p.njobs,
-                       p.l, p.js);
+    hipLaunchKernelGGL(k_pflags, dim3(p.jblocks ? p.jblocks : 1), dim3(kPrepBlock), 0, s, p.segs, p.nseg,
+                       nion, p.jseg, p.njobs, p.l, p.js);
     if ((e = hipGetLastError()) != hipSuccess)
         return e;
     hipLaunchKernelGGL(k_pscan, dim3(1), dim3(1024), 0, s, p.l.boff, nion);
     if ((e = hipGetLastError()) != hipSuccess)
         return e;
-    hipLaunchKernelGGL(k_pcompact, dim3(nion + ncell ? nion + ncell : 1), dim3(kPrepBlock), 0, s, p.segs, p.nseg,
-                       nion, p.l, p.centers);
-    if ((e = hipGetLastError()) != hipSuccess)
-        return e;
+    if (nion + ncell > 0) {
+        hipLaunchKernelGGL(k_pcompact, dim3(nion + ncell), dim3(kPrepBlock), 0, s, p.segs, nion,
+                           p.l, p.centers);
+        if ((e = hipGetLastError()) != hipSuccess)
+            return e;
+    }
     hipLaunchKernelGGL(k_pscan, dim3(1), dim3(1024), 0, s, p.l.toff, ncell);
     if ((e = hipGetLastError()) != hipSuccess)
         return e;
-    hipLaunchKernelGGL(k_ptilewrite, dim3(ncell ? ncell * kPrepItems : 1), dim3(kPrepBlock), 0, s,
-                       p.segs, p.nseg, p.jseg, p.njobs, p.l, p.tiles, p.js);
+    // workgroups for a block of the cell space: one per kPrepBlock of its cells,
+    // or, where these are more padding than cells and the blocks fill the device
+    // without, one
+    const uint32_t per = ncell > 1024u && 2 * p.nc < p.Ec ? 1u : (uint32_t)kPrepItems;
+    hipLaunchKernelGGL(k_ptilewrite, dim3(ncell ? ncell * per : 1), dim3(kPrepBlock), 0, s,
+                       p.segs, nion, ncell, per, p.jseg, p.njobs, p.l, p.tiles, p.js);
     return hipGetLastError();
 }
 
