@@ -33,7 +33,7 @@ sys.path.insert(0, ROOT)
 METRIC = "pair-distance evals/s at 20M ions; served jobs/s + p99 latency vs plain loop"
 FP32_PEAK_FLOPS = 157.3e12  # MI355X published FP32 vector peak (an FMA counts as 2 FLOP)
 VALU_PEAK_OPS = 78.6e12     # the same peak as FP32 element-ops (one FMA = one op)
-PLAIN_PEAK_OPS = 39.3e12    # without packed FP32: one wave-64 VALU instruction per CU per clock
+PLAIN_PEAK_OPS = 39.3e12    # one wave-64 VALU instruction per CU per clock (a scale, no ceiling: below)
 FLOP_PER_EVAL = 8           # 3 sub + 3 mul + 2 add (no FMA: fp-contract off)
 OPS_PER_EVAL = 9            # the same plus the in-ball compare
 # HBM bytes of the query kernel per step of the 20M-ion headline job, from two
@@ -41,9 +41,9 @@ OPS_PER_EVAL = 9            # the same plus the in-ball compare
 # factors a 1 GiB device copy reads): 48.4 GB read + 9.3 GB written
 TRAFFIC_HEADLINE = 5.78e10
 TRAFFIC_SOURCE = "profiles/k_query_frustum20M_rdf_mknn100.md"
-# the same for the 100M-ion job's query launches: 161.3 GB read + 11.9 GB
-# written
-TRAFFIC_LARGE = 1.732e11
+# the same for the 100M-ion job's query launches, its rerun's 17.8 GB left out:
+# 168.8 GB read + 11.9 GB written
+TRAFFIC_LARGE = 1.807e11
 TRAFFIC_LARGE_SOURCE = "profiles/k_query_frustum100M_rdf_mknn20.md"
 
 
@@ -89,9 +89,11 @@ def roofline(cand, kernel_ms, kernel, traffic=None, traffic_source=None):
         "frac_elementops": ops / (VALU_PEAK_OPS / 1e12),
         "frac_practical": ops / (PLAIN_PEAK_OPS / 1e12),
         "practical_note": "9 element-ops per evaluation (the 8 FLOP and the in-ball compare) "
-                          "against 78.6 T element-ops/s; packed FP32 (v_pk_*_f32) is disabled "
-                          "in this build, so plain FP32 issues one wave-64 instruction per CU "
-                          "per clock: 39.3 T element-ops/s is the practical ceiling",
+                          "against 39.3 T element-ops/s, one wave-64 instruction per CU per "
+                          "clock: what a probe reached for an FMA, a conversion and operands in "
+                          "scalar registers (0.9 to 1.0).  Sub, mul and add of vector registers "
+                          "reached 1.4 to 1.6, a compare 0.85, a square root 0.48, so this is a "
+                          "scale and no ceiling; packed FP32 is disabled in this build",
         "traffic": traffic,
         "traffic_unit": "bytes per step (HBM, all query launches)",
         "traffic_source": traffic_source,

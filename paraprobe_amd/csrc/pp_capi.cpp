@@ -913,7 +913,11 @@ void layout_prep_upload(PrepArena &a, Carver &m)
     a.segs = m.take<PrepSeg>((size_t)std::max(a.nseg, 1));
 }
 
-// Bytes of one job's share of a run's scratch (admission control).
+// Bytes of one job's share of a run's scratch, by which the serving loop admits
+// requests: for the lists the room of a 4-byte flag and position per ion and
+// segment and a count and offset per cell.  The lists take a small part of it
+// from some 50 ions a segment on; the figure stays, so that what a budget
+// admits and refuses stays.
 size_t prep_bytes(uint64_t n, uint64_t nc, int ntrg)
 {
     const uint64_t k = (uint64_t)std::max(ntrg, 1);
@@ -1208,7 +1212,7 @@ bool has_cross(const JobRun &r, int mode) { return mode != 1 && r.sym_minor != 0
 // fewer evaluations; whole calls: 4M ions, 9 type pairs, R 3 nm, pair counts 8.2
 // and 7.6 ms, with a row for both 6.78 and 6.63; 20M ions, R 5 nm, k to 100:
 // 151.1 and 148.3 ms).  Left out when the rows would cost resident workgroups
-// (100M ions, C 602: 349 ms of query kernel with five workgroups, 334 without
+// (100M ions, C 602: 306 ms of query kernel with five workgroups, 298 without
 // the rows and six), or when the in-ball total is counted pair by pair.
 // Neither of the two is taken where its layout with 32-bit counters, which
 // run_jobs asks of every job, would not fit the LDS: a job that runs without

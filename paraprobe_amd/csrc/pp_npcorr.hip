@@ -219,11 +219,10 @@ __global__ __launch_bounds__(256) void k_npcorr(NpcArgs a)
     // go to lanes (lane l < 25: the first range of row l, lane 25 + l: its
     // second) with an exclusive prefix of their lengths.  Long ranges are
     // walked one by one, 64 candidates a step; short ones (sparse type lists)
-    // as one concatenation, each lane finding its range by a binary search
-    // over the prefix.  The records of the next step are loaded while f runs
-    // on the current ones; the loads are unconditional (the last step loads
-    // its own records again), so that no branch joins paths with different
-    // loads in flight.
+    // as one concatenation, each lane finding its range by marks.  The records
+    // of the next step are loaded while f runs on the current ones; the loads
+    // are unconditional (the last step loads its own records again), so that no
+    // branch joins paths with different loads in flight.
     auto sweep = [&](const Rows &rw, const gnf4 *p, auto &&f) {
         const int src = lane >= 25 ? lane - 25 : lane;
         const uint32_t sb2 = __shfl(rw.b2, src, kWave), se2 = __shfl(rw.e2, src, kWave);
