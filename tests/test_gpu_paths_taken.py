@@ -72,6 +72,8 @@ KNN = [
     (PAIRS, 0.005, [64, 65, 100], 1, 1, 1),
     (PAIRS, 0.01, [3, 400], 1, 0, 0),
     (PAIRS, 0.0015, [1, 20], 1, 0, 0),
+    (PAIRS, 1.9 / 1014.5, [1, 20, 60], 1, 1, 0),  # 1,016 categories, 254 groups of 4
+    (PAIRS, 1.9 / 1015.5, [1, 20, 60], 1, 0, 0),
     (MIX, 0.02, [1, 150], 1, 0, 0),
 ]
 
@@ -81,7 +83,7 @@ def test_knn_way(ctx, capfd, monkeypatch, tasks, incr, ks, mode, entries, own):
     tip = synth.tip(6_007, 3, "frustum", 9.0, 5.0, 8.0, [0.6, 0.3, 0.1])
     ctx.set_knn_range(0)  # full-range histograms
     try:
-        job = Job(tasks, 0.0, incr, 1.9, FAM_RDF | FAM_MKNN, kvalues=ks)
+        job = Job(tasks, 0.0, float(np.float32(incr)), 1.9, FAM_RDF | FAM_MKNN, kvalues=ks)
         _, lines, _, _ = check(ctx, capfd, monkeypatch, tip, tip.ion2surf_sqr, job)
     finally:
         ctx.set_knn_range()
