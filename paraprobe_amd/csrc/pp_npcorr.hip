@@ -144,6 +144,9 @@ struct Rows {
     uint32_t b1, e1, b2, e2;  // up to two candidate index ranges of one stencil row
 };
 
+// ONE: R * R or a bucket's share of it is no normal number, and one bucket
+// holds every d2 > 0, so the whole ball is gathered.
+template <bool ONE>
 __global__ __launch_bounds__(256) void k_npcorr(NpcArgs a)
 {
     __shared__ uint4 s_buf[kWaves][kNpcCap];
@@ -190,7 +193,7 @@ __global__ __launch_bounds__(256) void k_npcorr(NpcArgs a)
         const float hy0 = fmaxf(0.0f, fmaxf(-ya, -yb)), hz0 = fmaxf(0.0f, fmaxf(-za, -zb));
         const float hy1 = fmaxf(ya, yb), hz1 = fmaxf(za, zb);
         const float hmin2 = hy0 * hy0 + hz0 * hz0, hmax2 = hy1 * hy1 + hz1 * hz1;
-        ro = fminf(ro * inv + 1e-4f, 1e9f);  // (a whole row, also where R * R overflows)
+        ro = ro * inv + 1e-4f;
         ri = fmaxf(ri * inv - 1e-4f, 0.0f);
         if (hmin2 > ro * ro)
             return rw;
@@ -408,14 +411,18 @@ __global__ __launch_bounds__(256) void k_npcorr(NpcArgs a)
         if (inb <= (uint32_t)kNpcCap) {
             // the selected bucket's candidates, ranked; they lie in the shell
             // of the bucket's distances
-            // (in FP64: v_rcp_f32 and v_sqrt_f32 take subnormal numbers for
-            // zero, which the width of a bucket is for Rmax near 1e-18)
-            const double bw = 1.0 / (double)inv_b2;
+            // (bucket b starts at sqrt(b) / 16 of the buckets' radius; the width
+            // of a bucket in d2 may be a subnormal number, which v_rcp_f32 and
+            // v_sqrt_f32 take for zero)
+            static_assert(kNpcBuckets == 256, "sqrt(b / kNpcBuckets) = sqrt(b) / 16");
+            const float r16 = (full ? a.maxlen : r1) * 0.0625f;
             const Rows shell =
-                rows_for(ecs, (float)(sqrt(bsel * bw) * (1.0 - 0x1p-12)),
-                         (bsel == kNpcBuckets - 1 && full)
-                             ? reach
-                             : (float)(sqrt((bsel + 1) * bw) * (1.0 + 0x1p-12)));
+                ONE ? rows_for(ecs, 0.0f, full ? reach : r1 * (1.0f + 0x1p-12f))
+                    : rows_for(ecs, __builtin_amdgcn_sqrtf((float)bsel) * r16 * (1.0f - 0x1p-12f),
+                               (bsel == kNpcBuckets - 1 && full)
+                                   ? reach
+                                   : __builtin_amdgcn_sqrtf((float)(bsel + 1)) * r16 *
+                                         (1.0f + 0x1p-12f));
             uint32_t cnt = 0;
             sweep(shell, ep, [&](const float4 &q, bool ok) {
                 float u = 0.f, v = 0.f, w = 0.f, d2 = 0.f;
@@ -508,7 +515,9 @@ hipError_t launch_npcorr(const NpcArgs &a, hipStream_t s)
     const uint64_t blocks = (a.n + kWaves - 1) / kWaves;
     if (blocks > 0x7FFFFFFFull)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_npcorr, dim3((unsigned)blocks), dim3(kBlock), 0, s, a);
+    const bool one = !(a.inv_bucket > 0.0f && a.inv_bucket < __builtin_inff());
+    hipLaunchKernelGGL((one ? k_npcorr<true> : k_npcorr<false>), dim3((unsigned)blocks),
+                       dim3(kBlock), 0, s, a);
     return hipGetLastError();
 }
 

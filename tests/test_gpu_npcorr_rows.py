@@ -23,7 +23,7 @@ def check(ctx, xyz, ty, tasks, R, width, K):
     assert np.array_equal(got, want)
 
 
-@pytest.mark.parametrize("scale", [7e-19, 1e-18, 1.3e-18, 1e-17, 1.0, 1e18, 1.2e19])
+@pytest.mark.parametrize("scale", [4e-19, 7e-19, 1e-18, 1.3e-18, 1e-17, 1.0, 1e18, 1.2e19])
 def test_scales(ctx, scale):
     """R * R from the subnormal numbers' edge to the largest floats; from 7e-19 to
     1.3e-18 the width of a distance bucket is subnormal."""
